@@ -44,6 +44,12 @@ __device__ __forceinline__ uint32_t phx_xcd_swizzle(uint32_t b, uint32_t nblocks
     return (b % XCD) * (nblocks / XCD) + b / XCD;
 }
 
+// The same for any block count: the first nblocks % 8 XCDs take one more.
+__device__ __forceinline__ uint32_t phx_xcd_swizzle_any(uint32_t b, uint32_t nblocks) {
+    const uint32_t XCD = 8, x = b % XCD, per = nblocks / XCD, more = nblocks % XCD;
+    return x * per + (x < more ? x : more) + b / XCD;
+}
+
 __device__ __forceinline__ uint32_t phx_pack_h2(float lo, float hi) {
     phx_h2 v;
     v.x = (_Float16)lo;   // v_cvt_f16_f32: round to nearest even
@@ -66,8 +72,18 @@ __device__ __forceinline__ void phx_splitk_reduce(const float *W, int32_t S, TO 
          gi += (int64_t)phx_block_count() * blockDim.x) {
         const int64_t e = gi * 4;
         const int64_t r = e / N, c = e % N;
+        // planes in batches of four loads in flight (one at a time, a launch
+        // of 16 planes waited for 16 memory latencies), added in plane order
         phx_f4 acc = *(const phx_f4 *)(W + e);
-        for (int32_t sp = 1; sp < S; ++sp) acc = acc + *(const phx_f4 *)(W + sp * plane + e);
+        int32_t sp = 1;
+        for (; sp + 4 <= S; sp += 4) {
+            phx_f4 v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = *(const phx_f4 *)(W + (sp + u) * plane + e);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) acc = acc + v[u];
+        }
+        for (; sp < S; ++sp) acc = acc + *(const phx_f4 *)(W + sp * plane + e);
         TO *dst = C + r * ldc + c;
         phx_f4 o = alpha * acc;
         if constexpr (sizeof(TO) == 4) {

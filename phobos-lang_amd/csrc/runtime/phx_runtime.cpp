@@ -462,28 +462,28 @@ static int s32_variant(int64_t M, int64_t N, int64_t K) {
 // to give its kernel's target number of workgroups, within its chunk-length
 // floor and at most PHX_SPLIT_MAX chunks (phx_geometry.h).  PHX_GEMM_SPLIT=<n> in the environment
 // forces n (1 turns the split off), for measurement.
-int gemm_split(phx_kernel k, int64_t M, int64_t N, int64_t K) {
+static int gemm_split_rule(phx_kernel k, int64_t M, int64_t N, int64_t K) {
+    if (k == PHX_GEMM_FP32 && s32_rule(M, N, K) != 0) return 1;  // a smaller tile instead
     const int64_t tiles = ((M + PHX_H_BM - 1) / PHX_H_BM) * ((N + PHX_H_BN - 1) / PHX_H_BN);
+    if (tiles >= PHX_SPLIT_MIN_TILES) return 1;
     const int64_t steps = (K + PHX_SPLIT_KSTEP - 1) / PHX_SPLIT_KSTEP;
-    int64_t sp;
-    phx_plan pin;
-    if (const char *env = getenv("PHX_GEMM_SPLIT")) {
-        sp = atoi(env);
-    } else if (pinned_plan(gemm_key(k, M, N, K), &pin)) {
-        sp = pin.splits;
-    } else {
-        if (k == PHX_GEMM_FP32 && s32_rule(M, N, K) != 0) return 1;  // a smaller tile instead
-        if (tiles >= PHX_SPLIT_MIN_TILES) return 1;
-        const bool f32 = k == PHX_GEMM_FP32;
-        const int64_t min_steps = f32                            ? PHX_SPLIT_MIN_STEPS_F32
-                                  : tiles >= PHX_SPLIT_WIDE_TILES ? PHX_SPLIT_MIN_STEPS_F16_WIDE
-                                                                  : PHX_SPLIT_MIN_STEPS_F16;
-        sp = (f32 ? PHX_SPLIT_TARGET_F32 : PHX_SPLIT_TARGET_F16) / tiles;
-        if (sp > steps / min_steps) sp = steps / min_steps;
-        if (sp > PHX_SPLIT_MAX) sp = PHX_SPLIT_MAX;
-    }
+    const bool f32 = k == PHX_GEMM_FP32;
+    const int64_t min_steps = f32                            ? PHX_SPLIT_MIN_STEPS_F32
+                              : tiles >= PHX_SPLIT_WIDE_TILES ? PHX_SPLIT_MIN_STEPS_F16_WIDE
+                                                              : PHX_SPLIT_MIN_STEPS_F16;
+    int64_t sp = (f32 ? PHX_SPLIT_TARGET_F32 : PHX_SPLIT_TARGET_F16) / tiles;
+    if (sp > steps / min_steps) sp = steps / min_steps;
+    if (sp > PHX_SPLIT_MAX) sp = PHX_SPLIT_MAX;
     // chunks of whole steps; drop chunks the rounding left empty
     return round_split(steps, sp);
+}
+
+int gemm_split(phx_kernel k, int64_t M, int64_t N, int64_t K) {
+    const int64_t steps = (K + PHX_SPLIT_KSTEP - 1) / PHX_SPLIT_KSTEP;
+    phx_plan pin;
+    if (const char *env = getenv("PHX_GEMM_SPLIT")) return round_split(steps, atoi(env));
+    if (pinned_plan(gemm_key(k, M, N, K), &pin)) return round_split(steps, pin.splits);
+    return gemm_split_rule(k, M, N, K);
 }
 
 // Whether a gemm_fp16tc_fp32acc launch runs the eight-wave kernels
@@ -517,23 +517,23 @@ size_t gemm_split_bytes(int64_t M, int64_t N, int sp) {
 }
 
 // The split-K launches over a caller-provided workspace of
-// gemm_split_bytes(M, N, sp) bytes: gemm_splitk over (tiles, sp) workgroups,
-// then gemm_splitk_reduce, both on stream s.
-int launch_gemm_split_ws(phx_kernel k, const Desc *t, int64_t M, int64_t N, int64_t K,
-                         float alpha, float beta, int sp, hipStream_t s, uint64_t ws) {
+// gemm_split_bytes(M, N, sp) bytes: entry (a gemm_splitk form over tm x tn
+// tiles, threads per workgroup) over (tiles, sp) workgroups, then
+// gemm_splitk_reduce, both on stream s.
+static int launch_gemm_split_ws(phx_kernel k, const char *entry, int64_t tm, int64_t tn,
+                                uint32_t threads, const Desc *t, int64_t M, int64_t N, int64_t K,
+                                float alpha, float beta, int sp, hipStream_t s, uint64_t ws) {
     const char *file = kSpecs[k].file;
     hipFunction_t fk, fr;
-    const bool w8 = gemm_w8(k, M, N, K);
-    if (int rc = aux_function(file, w8 ? "gemm_w8_splitk" : "gemm_splitk", &fk)) return rc;
+    if (int rc = aux_function(file, entry, &fk)) return rc;
     if (int rc = aux_function(file, "gemm_splitk_reduce", &fr)) return rc;
-    const int64_t tiles = ((M + PHX_H_BM - 1) / PHX_H_BM) * ((N + PHX_H_BN - 1) / PHX_H_BN);
+    const int64_t tiles = ((M + tm - 1) / tm) * ((N + tn - 1) / tn);
     uint64_t a = t[0].ptr, b = t[1].ptr, c = t[2].ptr;
     int64_t lda = t[0].stride[0], ldb = t[1].stride[0], ldc = t[2].stride[0];
     int64_t kchunk = split_chunk(K, sp);
     void *ka[] = {&a, &b, &ws, &lda, &ldb, &M, &N, &K, &kchunk};
-    hipError_t e = hipModuleLaunchKernel(fk, (uint32_t)tiles, (uint32_t)sp, 1,
-                                         w8 ? PHX_TC_W8_THREADS : PHX_H_THREADS, 1, 1, 0, s, ka,
-                                         nullptr);
+    hipError_t e = hipModuleLaunchKernel(fk, (uint32_t)tiles, (uint32_t)sp, 1, threads, 1, 1, 0,
+                                         s, ka, nullptr);
     if (e != hipSuccess) return hip_error(e, "hipModuleLaunchKernel(gemm_splitk)");
     int32_t s32 = sp;
     void *ra[] = {&ws, &s32, &c, &ldc, &M, &N, &alpha, &beta};
@@ -552,6 +552,83 @@ static int gemm_split_fit(phx_kernel k, int64_t M, int64_t N, int64_t K, size_t 
     if (sp < 2) return 1;
     const int64_t steps = (K + PHX_SPLIT_KSTEP - 1) / PHX_SPLIT_KSTEP;
     return fit_split(steps, sp, gemm_split_bytes(M, N, 1), cap);
+}
+
+// The tiles of the f16-operand GEMMs a launch without a plan of its own
+// chooses among, and what one costs on MI355X, in nanoseconds.  A launch of
+// tiles x splits workgroups runs ceil(workgroups / 256) rounds on the CUs: a
+// single round takes `round` plus `step` per 64 columns of its K chunk, of
+// which `idle` percent are left when few CUs are busy (less contention and,
+// for the big tiles, a higher clock); each of several rounds takes `round2`
+// plus `step2` (co-resident workgroups overlap).  Fitted to HIP event times
+// over K = 64 .. 4096 and 64^2 .. 4096^2 outputs, where the pick was the
+// fastest tile or within 10% of it: 1024^2 outputs 64 x 64 (gemm_fp16 at K
+// 1024 7.0 us against 22.8 for the 256 x 256 tile split 4 ways), 1280^2 128 x
+// 64 (10.6 against 22.4), 2048^2 128 x 128 (21.7 against 36.3), 3072^2 256 x
+// 256 (64.4 against 75.9).
+struct HTile {
+    const char *entry, *split_entry;
+    int64_t tm, tn;
+    int64_t round, step, idle, round2, step2;
+};
+static const HTile kH16Tiles[] = {
+    {"gemm", "gemm_splitk", 256, 256, 9500, 1720, 42, 9500, 1720},
+    {"gemm_m128", "gemm_m128_splitk", 128, 128, 3800, 487, 53, 3800, 460},
+    {"gemm_m128x64", "gemm_m128x64_splitk", 128, 64, 1900, 306, 72, 1900, 360},
+    {"gemm_m64", "gemm_m64_splitk", 64, 64, 1100, 210, 77, 1100, 215},
+};
+static const HTile kTcTiles[] = {
+    {"gemm_w8", "gemm_w8_splitk", 256, 256, 12500, 1900, 58, 12500, 1900},
+    {"gemm_m128", "gemm_m128_splitk", 128, 128, 5400, 857, 75, 3000, 690},
+    {"gemm_m128x64", "gemm_m128x64_splitk", 128, 64, 2600, 580, 68, 2600, 640},
+    {"gemm_m64", "gemm_m64_splitk", 64, 64, 1500, 370, 85, 1500, 350},
+};
+constexpr int kHTiles = 4;
+
+// Estimated nanoseconds of a launch on tile ti in sp K chunks.  A split adds
+// its reduce kernel: about 2.5 us and the f32 planes at 4 TB/s.
+static int64_t htile_cost(const HTile &ti, int64_t M, int64_t N, int64_t K, int sp) {
+    const int64_t wgs = ((M + ti.tm - 1) / ti.tm) * ((N + ti.tn - 1) / ti.tn) * sp;
+    const int64_t steps = (split_chunk(K, sp) + 63) / 64;
+    int64_t ns = 2600;
+    if (wgs <= 256)
+        ns += ti.round + steps * ti.step * (ti.idle + (100 - ti.idle) * wgs / 256) / 100;
+    else
+        ns += (wgs + 255) / 256 * (ti.round2 + steps * ti.step2);
+    if (sp > 1) ns += 2500 + (sp + 1) * M * N / 1000;
+    return ns;
+}
+
+// The tile and K split of a gemm_fp16 or gemm_fp16tc_fp32acc launch that
+// follows the built-in plan: the cheapest of every tile in every split up to
+// max_sp chunks (the built-in plan's, cut to the bound workspace).
+static const HTile *gemm_tile_plan(phx_kernel k, int64_t M, int64_t N, int64_t K, int max_sp,
+                                   int *splits) {
+    const HTile *tiles = k == PHX_GEMM_FP16 ? kH16Tiles : kTcTiles;
+    const int64_t units = (K + PHX_SPLIT_KSTEP - 1) / PHX_SPLIT_KSTEP;
+    const HTile *best = nullptr;
+    int64_t least = 0;
+    for (int i = 0; i < kHTiles; ++i)
+        for (int want = 1; want <= max_sp; ++want) {
+            const int sp = round_split(units, want);
+            const int64_t ns = htile_cost(tiles[i], M, N, K, sp);
+            if (!best || ns < least) {
+                best = &tiles[i];
+                least = ns;
+                *splits = sp;
+            }
+        }
+    return best;
+}
+
+// Whether a launch follows the built-in plan: no environment variable forces
+// one, and none is pinned or the pinned one is the built-in rule's own.
+static bool gemm_follows_rule(phx_kernel k, int64_t M, int64_t N, int64_t K) {
+    if (getenv("PHX_GEMM_SPLIT") || getenv("PHX_GEMM_W8")) return false;
+    phx_plan pin;
+    if (!pinned_plan(gemm_key(k, M, N, K), &pin)) return true;
+    const int64_t units = (K + PHX_SPLIT_KSTEP - 1) / PHX_SPLIT_KSTEP;
+    return pin.variant == 0 && round_split(units, pin.splits) == gemm_split_rule(k, M, N, K);
 }
 
 // How many key chunks a flash launch is split into (1: no split).
@@ -627,6 +704,28 @@ static int flash_split_fit(phx_kernel k, int64_t BH, int64_t Nq, int64_t Nk, siz
     return fit_split(nkb, sp, flash_split_bytes(BH, Nq, 1), cap);
 }
 
+// One workgroup of `threads` per tm x tn output tile of a GEMM entry that
+// takes the .ph kernel's own argument list.
+static int launch_tiled(const char *file, const char *entry, int64_t tm, int64_t tn,
+                        uint32_t threads, int64_t M, int64_t N, hipStream_t s, void **args) {
+    hipFunction_t f;
+    if (int rc = aux_function(file, entry, &f)) return rc;
+    const uint32_t tiles = (uint32_t)(((M + tm - 1) / tm) * ((N + tn - 1) / tn));
+    hipError_t e = hipModuleLaunchKernel(f, tiles, 1, 1, threads, 1, 1, 0, s, args, nullptr);
+    return e == hipSuccess ? PHX_OK : hip_error(e, "hipModuleLaunchKernel(gemm tile)");
+}
+
+// Whether every GEMM operand's rows follow each other without overlap and
+// 257 of them span less than 2 GiB, which the smaller tiles assume (the
+// 256 x 256 kernels take what is left).
+static bool dense_rows(const Desc *t, const int64_t *d) {
+    const int64_t cols[3] = {d[2], d[1], d[1]};  // A, B, C of M x N x K
+    for (int i = 0; i < 3; ++i)
+        if (t[i].stride[0] < cols[i] || (PHX_H_BM + 1) * t[i].stride[0] * 4 > INT32_MAX)
+            return false;
+    return true;
+}
+
 int launch_raw(hipFunction_t f, const uint32_t grid[3], const uint32_t block[3], uint32_t shmem,
                hipStream_t s, void **args) {
     // A built-in kernel runs on this backend's own tiling, whatever geometry
@@ -650,36 +749,40 @@ int launch_raw(hipFunction_t f, const uint32_t grid[3], const uint32_t block[3],
                                  gemm_split((phx_kernel)k, d[0], d[1], d[2]) > 1 &&
                                  !pinned_plan(gemm_key((phx_kernel)k, d[0], d[1], d[2]), nullptr) &&
                                  !getenv("PHX_GEMM_SPLIT");
+            float alpha, beta;  // the two f32 scalars after the three memrefs
+            memcpy(&alpha, args[21], 4);
+            memcpy(&beta, args[22], 4);
+            if (k != PHX_GEMM_FP32 && gemm_follows_rule((phx_kernel)k, d[0], d[1], d[2]) &&
+                dense_rows(t, d)) {
+                int msp = 1;
+                const HTile *ti = gemm_tile_plan((phx_kernel)k, d[0], d[1], d[2], sp, &msp);
+                if (ti->tm < PHX_H_BM) {
+                    if (msp > 1)
+                        return launch_gemm_split_ws((phx_kernel)k, ti->split_entry, ti->tm, ti->tn,
+                                                    PHX_H_THREADS, t, d[0], d[1], d[2], alpha,
+                                                    beta, msp, s, w.ptr);
+                    return launch_tiled(kSpecs[k].file, ti->entry, ti->tm, ti->tn, PHX_H_THREADS,
+                                        d[0], d[1], s, args);
+                }
+            }
             if (sp > 1) {
-                float alpha, beta;  // the two f32 scalars after the three memrefs
-                memcpy(&alpha, args[21], 4);
-                memcpy(&beta, args[22], 4);
-                return launch_gemm_split_ws((phx_kernel)k, t, d[0], d[1], d[2], alpha, beta, sp,
-                                            s, w.ptr);
+                const bool w8 = gemm_w8((phx_kernel)k, d[0], d[1], d[2]);
+                return launch_gemm_split_ws((phx_kernel)k, w8 ? "gemm_w8_splitk" : "gemm_splitk",
+                                            PHX_H_BM, PHX_H_BN,
+                                            w8 ? PHX_TC_W8_THREADS : PHX_H_THREADS, t, d[0], d[1],
+                                            d[2], alpha, beta, sp, s, w.ptr);
             }
             if (k == PHX_GEMM_FP32) {
                 const int v = no_room ? PHX_S32_SMALL_VARIANT : s32_variant(d[0], d[1], d[2]);
                 if (v) {
                     const S32Tiling &ti = kS32[v];
-                    hipFunction_t fv;
-                    if (int rc = aux_function(kSpecs[k].file, ti.entry, &fv)) return rc;
-                    const uint32_t tiles = (uint32_t)(((d[0] + ti.tm - 1) / ti.tm) *
-                                                      ((d[1] + ti.tn - 1) / ti.tn));
-                    hipError_t e = hipModuleLaunchKernel(fv, tiles, 1, 1, PHX_S_THREADS, 1, 1, 0,
-                                                         s, args, nullptr);
-                    if (e != hipSuccess) return hip_error(e, "hipModuleLaunchKernel(gemm tiling)");
-                    return PHX_OK;
+                    return launch_tiled(kSpecs[k].file, ti.entry, ti.tm, ti.tn, PHX_S_THREADS,
+                                        d[0], d[1], s, args);
                 }
             }
             if (gemm_w8((phx_kernel)k, d[0], d[1], d[2])) {
-                hipFunction_t fw;
-                if (int rc = aux_function(kSpecs[k].file, "gemm_w8", &fw)) return rc;
-                const uint32_t tiles = (uint32_t)(((d[0] + PHX_H_BM - 1) / PHX_H_BM) *
-                                                  ((d[1] + PHX_H_BN - 1) / PHX_H_BN));
-                hipError_t e = hipModuleLaunchKernel(fw, tiles, 1, 1, PHX_TC_W8_THREADS, 1, 1, 0,
-                                                     s, args, nullptr);
-                if (e != hipSuccess) return hip_error(e, "hipModuleLaunchKernel(gemm_w8)");
-                return PHX_OK;
+                return launch_tiled(kSpecs[k].file, "gemm_w8", PHX_H_BM, PHX_H_BN,
+                                    PHX_TC_W8_THREADS, d[0], d[1], s, args);
             }
         }
         if (k == PHX_FLASH_FP16 || k == PHX_FLASH_FP32 || k == PHX_FLASH_FP16_BH ||
