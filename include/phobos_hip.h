@@ -103,8 +103,7 @@ int phx_stream_synchronize(phx_stream s);
  * engine.rs:582-647) for the split launches of this backend.  A built-in
  * GEMM or flash launch that phx_split_plan would split runs with the largest
  * split whose workspace fits in the bound bytes, and unsplit when none fits
- * or nothing is bound (gemm_fp32 without a pin then takes its 64 x 64 x 16
- * tiling, which needs no workspace); it never allocates.  The buffer must stay valid until
+ * or nothing is bound; it never allocates.  The buffer must stay valid until
  * every launch on s that may use it has completed; launches on one stream
  * run in order, so they can share it.  Unbinding (or phx_stream_destroy)
  * forgets it; the caller frees it. */
@@ -170,11 +169,10 @@ int phx_check_shape(phx_kernel k, const int64_t *dims, int ndims);
  * whose bound workspace holds at least *workspace_bytes: *splits K
  * chunks (gemm_fp32, gemm_fp16tc_fp32acc, gemm_fp16) or key chunks (flash),
  * 1 for none, and the workspace bytes that needs (0 for none).  With a
- * smaller workspace a launch takes fewer chunks, down to none.  For
- * gemm_fp16tc_fp32acc and gemm_fp16 it is the split of the 256 x 256 tile
- * and the most a launch uses: one that follows the built-in plan runs a
- * smaller output tile instead, with fewer chunks or none, where that is
- * faster.  Other
+ * smaller workspace a launch takes fewer chunks, down to none.  For the
+ * GEMMs it is the split of the 256 x 256 tile and the most a launch uses:
+ * one that follows the built-in plan runs a smaller output tile instead, with
+ * fewer chunks or none, where that is faster.  Other
  * kernels never split.  No counterpart in the reference, whose autotuner
  * picks tile sizes instead (phobos-bench/src/autotune.rs:98-192). */
 int phx_split_plan(phx_kernel k, const int64_t *dims, int ndims, int *splits,
@@ -197,11 +195,12 @@ int phx_split_plan(phx_kernel k, const int64_t *dims, int ndims, int *splits,
  *            "gemm_w8", "gemm_w8_splitk"), 1 the one-wave kernels ("gemm",
  *            "gemm_splitk"), split or not; 0 for every other kernel.
  * A launch uses the plan pinned for its kernel and dims, else the built-in
- * rule.  gemm_fp16tc_fp32acc and gemm_fp16 launches under the built-in rule,
- * or under a pin equal to it, may run a smaller output tile (64 x 64, 128 x
- * 64 or 128 x 128: entries "gemm_m64", "gemm_m128x64", "gemm_m128" and their
- * "_splitk" forms) with at most the rule's chunks; any other pin runs the 256
- * x 256 tile.  The PHX_GEMM_SPLIT, PHX_FLASH_SPLIT and PHX_GEMM_W8 environment
+ * rule.  GEMM launches under the built-in rule, or under a pin equal to it,
+ * may run a smaller output tile with at most the rule's chunks
+ * (gemm_fp16tc_fp32acc and gemm_fp16: 64 x 64, 128 x 64 or 128 x 128, entries
+ * "gemm_m64", "gemm_m128x64", "gemm_m128"; gemm_fp32: 64 x 64, 64 x 32 or 32 x
+ * 32, entries "gemm_s64", "gemm_s64x32", "gemm_s32"; and their "_splitk"
+ * forms); any other pin runs the tile it names.  The PHX_GEMM_SPLIT, PHX_FLASH_SPLIT and PHX_GEMM_W8 environment
  * variables, which force a plan for measurement, take precedence over both. */
 typedef struct {
     int32_t splits;

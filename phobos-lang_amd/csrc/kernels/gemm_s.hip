@@ -375,16 +375,54 @@ __device__ __forceinline__ void gemm_s_body(const float *A, int64_t lda, const f
 
 typedef Tile<PHX_S_TILE, PHX_S_TILE, PHX_S_BK> Base;  // 256 x 256 x 16
 
+// Operands the kernels do not take (the host refuses them before a launch).
+#define GEMM_S_REFUSED                                                                        \
+    (blockDim.x != NT || N % PHX_S_NK_MULT || K % PHX_S_NK_MULT || M <= 0 || N <= 0 ||       \
+     K <= 0 || b_s0 != K || c_s0 != M || c_s1 != N || a_st1 != 1 || b_st1 != 1 ||            \
+     c_st1 != 1 || (a_st0 | b_st0 | c_st0) % 4 ||                                            \
+     ((uintptr_t)(a_ptr + a_off) | (uintptr_t)(b_ptr + b_off) | (uintptr_t)(c_ptr + c_off)) & 15)
+
 #define GEMM_S_PRELUDE(T)                                                                     \
     __shared__ __attribute__((aligned(16))) char stg[NSTG * T::STAGE];                        \
     const int64_t M = a_s0, K = a_s1, N = b_s1;                                               \
-    if (blockDim.x != NT || N % PHX_S_NK_MULT || K % PHX_S_NK_MULT || M <= 0 || N <= 0 ||  \
-        K <= 0 || b_s0 != K || c_s0 != M || c_s1 != N || a_st1 != 1 || b_st1 != 1 ||         \
-        c_st1 != 1 || (a_st0 | b_st0 | c_st0) % 4 ||                                         \
-        ((uintptr_t)(a_ptr + a_off) | (uintptr_t)(b_ptr + b_off) | (uintptr_t)(c_ptr + c_off)) & 15) \
-        return;
+    if (GEMM_S_REFUSED) return;
+
+// ------------------------------------------------------ smaller tiles
+#include "gemm_s_tiles.h"
+typedef STile<2, 2, 32> S64;
+typedef STile<2, 1, 32> S64x32;
+typedef STile<1, 1, 64> S32;
+
+#define GEMM_S_TILE_ENTRY(NAME, T, BETA)                                                      \
+    extern "C" __global__ __launch_bounds__(NT, 3) void NAME(                                 \
+        PHX_MEMREF2(float, a, int32_t), PHX_MEMREF2(float, b, int32_t),                       \
+        PHX_MEMREF2(float, c, int32_t), float alpha, float beta) {                            \
+        const int64_t M = a_s0, K = a_s1, N = b_s1;                                           \
+        if (GEMM_S_REFUSED || a_st0 < K || b_st0 < N || c_st0 < N) return;                    \
+        s_body<T>(a_ptr + a_off, a_st0, b_ptr + b_off, b_st0, c_ptr + c_off, c_st0, M, N, K,  \
+                  alpha, BETA, phx_block_linear(), phx_block_count());                        \
+    }
 
 #ifdef PHX_GEMM_FP32
+GEMM_S_TILE_ENTRY(gemm_s64, S64, beta)
+GEMM_S_TILE_ENTRY(gemm_s64x32, S64x32, beta)
+GEMM_S_TILE_ENTRY(gemm_s32, S32, beta)
+
+// Their split-K forms, as gemm_splitk below.
+#define GEMM_S_TILE_SPLIT(NAME, T)                                                            \
+    extern "C" __global__ __launch_bounds__(NT, 3) void NAME(                                 \
+        const float *A, const float *B, float *W, int64_t lda, int64_t ldb, int64_t M,        \
+        int64_t N, int64_t K, int64_t kchunk) {                                               \
+        const int64_t k0 = (int64_t)blockIdx.y * kchunk;                                      \
+        if (blockDim.x != NT || k0 >= K || kchunk % Base::TK) return;                         \
+        const int64_t kc = K - k0 < kchunk ? K - k0 : kchunk;                                 \
+        s_body<T>(A + k0, lda, B + k0 * ldb, ldb, W + (int64_t)blockIdx.y * M * N, N, M, N,   \
+                  kc, 1.0f, 0.0f, blockIdx.x, gridDim.x);                                     \
+    }
+GEMM_S_TILE_SPLIT(gemm_s64_splitk, S64)
+GEMM_S_TILE_SPLIT(gemm_s64x32_splitk, S64x32)
+GEMM_S_TILE_SPLIT(gemm_s32_splitk, S32)
+
 extern "C" __global__ __launch_bounds__(NT, 1) void gemm(PHX_MEMREF2(float, a, int32_t),
                                                           PHX_MEMREF2(float, b, int32_t),
                                                           PHX_MEMREF2(float, c, int32_t),
@@ -449,6 +487,11 @@ extern "C" __global__ __launch_bounds__(256) void gemm_splitk_reduce(const float
 #endif
 
 #ifdef PHX_MATMUL_CLUSTER
+// C = fl(fl(alpha*acc) + c_old): beta 1, which multiplies c_old exactly
+GEMM_S_TILE_ENTRY(matmul_s64, S64, 1.0f)
+GEMM_S_TILE_ENTRY(matmul_s64x32, S64x32, 1.0f)
+GEMM_S_TILE_ENTRY(matmul_s32, S32, 1.0f)
+
 extern "C" __global__ __launch_bounds__(NT, 1) void matmul(PHX_MEMREF2(float, a, int32_t),
                                                             PHX_MEMREF2(float, b, int32_t),
                                                             PHX_MEMREF2(float, c, int32_t),

@@ -621,6 +621,58 @@ static const HTile *gemm_tile_plan(phx_kernel k, int64_t M, int64_t N, int64_t K
     return best;
 }
 
+// The tiles of the f32 GEMMs (gemm_fp32 under the built-in plan, and the
+// cluster step leaf, which has no plan), and what one costs on MI355X in
+// nanoseconds: the fullest CU takes ceil(workgroups / 256) of them, three at
+// a time, each `round` plus, per 64 columns of its K chunk, step[0], [1] or
+// [2] for one, two or three together (alone, a workgroup's one wave per SIMD
+// leaves latencies open).  Fitted to HIP event times at 64 .. 4096 (within
+// 8%): 512^3 runs 32 x 32 (5.3 us against 12.4 for the 64 x 64 x 16 tiling,
+// 7.1 for 64 x 32), 1024^3 64 x 64 (18.7 against 22.2; 21.8 for 32 x 32), 1200
+// x 2000 x 1000 64 x 32 (42.8 against 52; 47.2 for 64 x 64), 4096^3 256 x 256
+// (926; 945 for 64 x 64).
+struct SHTile {
+    const char *entry, *split_entry, *leaf;
+    int64_t tm, tn, round, step[3];
+};
+static const SHTile kSTiles[] = {
+    {"gemm", "gemm_splitk", "matmul", 256, 256, 8000, {14200, 28400, 42600}},
+    {"gemm_s64", "gemm_s64_splitk", "matmul_s64", 64, 64, 800, {930, 1800, 2680}},
+    {"gemm_s64x32", "gemm_s64x32_splitk", "matmul_s64x32", 64, 32, 600, {780, 1140, 1380}},
+    {"gemm_s32", "gemm_s32_splitk", "matmul_s32", 32, 32, 550, {370, 560, 780}},
+};
+// Workgroups a small f32 tile's launch starts at most, walking the tiles with
+// that stride: the three per CU that are resident at once (at 2048^3 the 64 x
+// 64 tile took 148 us with a workgroup per tile, 121 so).
+constexpr uint32_t kSTileGrid = 768;
+
+static int64_t stile_cost(const SHTile &ti, int64_t M, int64_t N, int64_t K, int sp) {
+    const int64_t wgs = ((M + ti.tm - 1) / ti.tm) * ((N + ti.tn - 1) / ti.tn) * sp;
+    const int64_t steps = (split_chunk(K, sp) + 63) / 64;
+    const int64_t n = (wgs + 255) / 256;
+    int64_t ns = 2600 + n * ti.round + n / 3 * steps * ti.step[2];
+    if (n % 3) ns += steps * ti.step[n % 3 - 1];
+    if (sp > 1) ns += 2500 + (sp + 1) * M * N / 1000;  // the reduce kernel
+    return ns;
+}
+
+static const SHTile *s_tile_plan(int64_t M, int64_t N, int64_t K, int max_sp, int *splits) {
+    const int64_t units = (K + PHX_SPLIT_KSTEP - 1) / PHX_SPLIT_KSTEP;
+    const SHTile *best = nullptr;
+    int64_t least = 0;
+    for (const SHTile &ti : kSTiles)
+        for (int want = 1; want <= max_sp; ++want) {
+            const int sp = round_split(units, want);
+            const int64_t ns = stile_cost(ti, M, N, K, sp);
+            if (!best || ns < least) {
+                best = &ti;
+                least = ns;
+                *splits = sp;
+            }
+        }
+    return best;
+}
+
 // Whether a launch follows the built-in plan: no environment variable forces
 // one, and none is pinned or the pinned one is the built-in rule's own.
 static bool gemm_follows_rule(phx_kernel k, int64_t M, int64_t N, int64_t K) {
@@ -628,7 +680,9 @@ static bool gemm_follows_rule(phx_kernel k, int64_t M, int64_t N, int64_t K) {
     phx_plan pin;
     if (!pinned_plan(gemm_key(k, M, N, K), &pin)) return true;
     const int64_t units = (K + PHX_SPLIT_KSTEP - 1) / PHX_SPLIT_KSTEP;
-    return pin.variant == 0 && round_split(units, pin.splits) == gemm_split_rule(k, M, N, K);
+    const int sp = gemm_split_rule(k, M, N, K);
+    const int variant = k == PHX_GEMM_FP32 && sp == 1 ? s32_rule(M, N, K) : 0;
+    return pin.variant == variant && round_split(units, pin.splits) == sp;
 }
 
 // How many key chunks a flash launch is split into (1: no split).
@@ -704,14 +758,16 @@ static int flash_split_fit(phx_kernel k, int64_t BH, int64_t Nq, int64_t Nk, siz
     return fit_split(nkb, sp, flash_split_bytes(BH, Nq, 1), cap);
 }
 
-// One workgroup of `threads` per tm x tn output tile of a GEMM entry that
-// takes the .ph kernel's own argument list.
+// One workgroup of `threads` per tm x tn output tile, at most cap of them
+// (0: any number), of a GEMM entry that takes the .ph kernel's own argument
+// list and walks the tiles with the grid's stride.
 static int launch_tiled(const char *file, const char *entry, int64_t tm, int64_t tn,
-                        uint32_t threads, int64_t M, int64_t N, hipStream_t s, void **args) {
+                        uint32_t threads, uint32_t cap, int64_t M, int64_t N, hipStream_t s, void **args) {
     hipFunction_t f;
     if (int rc = aux_function(file, entry, &f)) return rc;
-    const uint32_t tiles = (uint32_t)(((M + tm - 1) / tm) * ((N + tn - 1) / tn));
-    hipError_t e = hipModuleLaunchKernel(f, tiles, 1, 1, threads, 1, 1, 0, s, args, nullptr);
+    const int64_t tiles = ((M + tm - 1) / tm) * ((N + tn - 1) / tn);
+    const uint32_t grid = (uint32_t)(cap && tiles > cap ? cap : tiles);
+    hipError_t e = hipModuleLaunchKernel(f, grid, 1, 1, threads, 1, 1, 0, s, args, nullptr);
     return e == hipSuccess ? PHX_OK : hip_error(e, "hipModuleLaunchKernel(gemm tile)");
 }
 
@@ -742,28 +798,33 @@ int launch_raw(hipFunction_t f, const uint32_t grid[3], const uint32_t block[3],
             if (int rc = check_shape((phx_kernel)k, d, nd)) return rc;
             const Workspace w = stream_workspace(s);
             const int sp = gemm_split_fit((phx_kernel)k, d[0], d[1], d[2], w.bytes);
-            // gemm_fp32's built-in plan split over K, but the stream has no
-            // workspace for it: the 64 x 64 tiling fills the GPU without one
-            // (256^2 x 8192: 151 us against 1.8 ms for one 256 x 256 tile)
-            const bool no_room = k == PHX_GEMM_FP32 && sp == 1 &&
-                                 gemm_split((phx_kernel)k, d[0], d[1], d[2]) > 1 &&
-                                 !pinned_plan(gemm_key((phx_kernel)k, d[0], d[1], d[2]), nullptr) &&
-                                 !getenv("PHX_GEMM_SPLIT");
             float alpha, beta;  // the two f32 scalars after the three memrefs
             memcpy(&alpha, args[21], 4);
             memcpy(&beta, args[22], 4);
-            if (k != PHX_GEMM_FP32 && gemm_follows_rule((phx_kernel)k, d[0], d[1], d[2]) &&
-                dense_rows(t, d)) {
+            if (gemm_follows_rule((phx_kernel)k, d[0], d[1], d[2]) && dense_rows(t, d)) {
                 int msp = 1;
-                const HTile *ti = gemm_tile_plan((phx_kernel)k, d[0], d[1], d[2], sp, &msp);
-                if (ti->tm < PHX_H_BM) {
+                const char *entry, *split_entry;
+                int64_t tm, tn;
+                uint32_t cap = 0;
+                if (k == PHX_GEMM_FP32) {
+                    const SHTile *ti = s_tile_plan(d[0], d[1], d[2], sp, &msp);
+                    entry = ti->entry, split_entry = ti->split_entry, tm = ti->tm, tn = ti->tn;
+                    cap = kSTileGrid;
+                } else {
+                    const HTile *ti = gemm_tile_plan((phx_kernel)k, d[0], d[1], d[2], sp, &msp);
+                    entry = ti->entry, split_entry = ti->split_entry, tm = ti->tm, tn = ti->tn;
+                }
+                if (tm < PHX_H_BM) {
                     if (msp > 1)
-                        return launch_gemm_split_ws((phx_kernel)k, ti->split_entry, ti->tm, ti->tn,
+                        return launch_gemm_split_ws((phx_kernel)k, split_entry, tm, tn,
                                                     PHX_H_THREADS, t, d[0], d[1], d[2], alpha,
                                                     beta, msp, s, w.ptr);
-                    return launch_tiled(kSpecs[k].file, ti->entry, ti->tm, ti->tn, PHX_H_THREADS,
-                                        d[0], d[1], s, args);
+                    return launch_tiled(kSpecs[k].file, entry, tm, tn, PHX_H_THREADS, cap, d[0],
+                                        d[1], s, args);
                 }
+                if (k == PHX_GEMM_FP32 && msp == 1)
+                    return launch_tiled(kSpecs[k].file, entry, tm, tn, PHX_S_THREADS, 0, d[0],
+                                        d[1], s, args);
             }
             if (sp > 1) {
                 const bool w8 = gemm_w8((phx_kernel)k, d[0], d[1], d[2]);
@@ -773,17 +834,32 @@ int launch_raw(hipFunction_t f, const uint32_t grid[3], const uint32_t block[3],
                                             d[2], alpha, beta, sp, s, w.ptr);
             }
             if (k == PHX_GEMM_FP32) {
+                // a built-in plan that splits, without a workspace for it (rows
+                // the small tiles do not take): the 64 x 64 x 16 tiling fills
+                // the GPU without one (256^2 x 8192: 151 us against 1.8 ms for
+                // one 256 x 256 tile)
+                const bool no_room =
+                    gemm_split((phx_kernel)k, d[0], d[1], d[2]) > 1 &&
+                    !pinned_plan(gemm_key((phx_kernel)k, d[0], d[1], d[2]), nullptr) &&
+                    !getenv("PHX_GEMM_SPLIT");
                 const int v = no_room ? PHX_S32_SMALL_VARIANT : s32_variant(d[0], d[1], d[2]);
                 if (v) {
                     const S32Tiling &ti = kS32[v];
-                    return launch_tiled(kSpecs[k].file, ti.entry, ti.tm, ti.tn, PHX_S_THREADS,
+                    return launch_tiled(kSpecs[k].file, ti.entry, ti.tm, ti.tn, PHX_S_THREADS, 0,
                                         d[0], d[1], s, args);
                 }
             }
-            if (gemm_w8((phx_kernel)k, d[0], d[1], d[2])) {
+            if (gemm_w8((phx_kernel)k, d[0], d[1], d[2]))
                 return launch_tiled(kSpecs[k].file, "gemm_w8", PHX_H_BM, PHX_H_BN,
-                                    PHX_TC_W8_THREADS, d[0], d[1], s, args);
-            }
+                                    PHX_TC_W8_THREADS, 0, d[0], d[1], s, args);
+        }
+        if (k == PHX_MATMUL) {
+            if (int rc = check_shape((phx_kernel)k, d, nd)) return rc;
+            int msp = 1;
+            const SHTile *ti = s_tile_plan(d[0], d[1], d[2], 1, &msp);
+            if (ti->tm < PHX_S_TILE && dense_rows(t, d))
+                return launch_tiled(kSpecs[k].file, ti->leaf, ti->tm, ti->tn, PHX_S_THREADS,
+                                    kSTileGrid, d[0], d[1], s, args);
         }
         if (k == PHX_FLASH_FP16 || k == PHX_FLASH_FP32 || k == PHX_FLASH_FP16_BH ||
             k == PHX_FLASH_FP32_BH) {

@@ -1,6 +1,6 @@
-"""The smaller output tiles of gemm_fp16 and gemm_fp16tc_fp32acc
-(csrc/kernels/gemm_tiles.h: gemm_m64, gemm_m128x64, gemm_m128 and their
-split-K forms) at the edges of their tiles.
+"""The smaller output tiles of the GEMMs at the edges of their tiles:
+gemm_fp16 and gemm_fp16tc_fp32acc (csrc/kernels/gemm_tiles.h), gemm_fp32 and
+the cluster step leaf (gemm_s_tiles.h), and their split-K forms.
 
 An output is an f32 sum of K exact products in some order, so it lies within
 K eps of the sum of their magnitudes (K * 2^-24 * |A|@|B|) of the f64 oracle,
@@ -18,8 +18,12 @@ import oracle
 
 pytestmark = pytest.mark.gpu
 
-ENTRIES = {"gemm_m64": (64, 64), "gemm_m128x64": (128, 64), "gemm_m128": (128, 128)}
-KERNELS = {"GEMM_FP16": "gemm_fp16.hsaco", "GEMM_FP16TC_FP32ACC": "gemm_fp16tc_fp32acc.hsaco"}
+M_ENTRIES = {"gemm_m64": (64, 64), "gemm_m128x64": (128, 64), "gemm_m128": (128, 128)}
+S_ENTRIES = {"s64": (64, 64), "s64x32": (64, 32), "s32": (32, 32)}
+KERNELS = {"GEMM_FP16": ("gemm_fp16.hsaco", M_ENTRIES),
+           "GEMM_FP16TC_FP32ACC": ("gemm_fp16tc_fp32acc.hsaco", M_ENTRIES),
+           "GEMM_FP32": ("gemm_fp32.hsaco", {"gemm_" + n: t for n, t in S_ENTRIES.items()}),
+           "MATMUL": ("matmul_cluster_fp32.hsaco", {"matmul_" + n: t for n, t in S_ENTRIES.items()})}
 # one row and the smallest N and K, whole tiles, one past a tile, one K step
 # and one past it, a K of every stage of the rings, a partial last K step
 SHAPES = [(1, 8, 8), (64, 64, 64), (65, 72, 72), (128, 128, 128), (129, 136, 200),
@@ -33,6 +37,7 @@ class _Case:
     def __init__(self, px, kern, M, N, K, pad, seed=5):
         self.px, self.kern, self.dims = px, kern, (M, N, K)
         self.f16 = kern == px.GEMM_FP16
+        self.idx = ctypes.c_int32 if kern in (px.GEMM_FP32, px.MATMUL) else ctypes.c_int64
         A = oracle.f16_round(oracle.normal_f32(seed, M * K, 1 / np.sqrt(K))).reshape(M, K)
         B = oracle.f16_round(oracle.normal_f32(seed + 1, K * N, 1 / np.sqrt(K))).reshape(K, N)
         C = oracle.f16_round(oracle.normal_f32(seed + 2, M * N)).reshape(M, N)
@@ -51,7 +56,7 @@ class _Case:
         vals = []
         for t, buf, (r, c) in zip(self.host, self.dev, (self.A.shape, self.B.shape, self.C.shape)):
             vals += [ctypes.c_uint64(buf.ptr), ctypes.c_uint64(buf.ptr)]
-            vals += [ctypes.c_int64(v) for v in (0, r, c, t.shape[1], 1)]
+            vals += [self.idx(v) for v in (0, r, c, t.shape[1], 1)]
         vals += [ctypes.c_float(alpha), ctypes.c_float(beta)]
         return vals, (ctypes.c_void_p * len(vals))(
             *[ctypes.cast(ctypes.byref(v), ctypes.c_void_p) for v in vals])
@@ -74,6 +79,8 @@ class _Case:
 
 
 def _check(case, bits, alpha, beta):
+    if case.kern == case.px.MATMUL:
+        beta = 1.0  # the step leaf's, whatever it is passed
     got = case.values(bits).reshape(case.C.shape)
     ref = oracle.gemm_full(case.A, case.B, case.C, alpha, beta, round16=True)
     K = case.dims[2]
@@ -92,22 +99,23 @@ def test_each_tile_meets_the_oracle(px_gpu, stream, kern_name, M, N, K, pad):
     # workgroups than tiles (the block-stride walk), C read and not read
     px = px_gpu
     case = _Case(px, getattr(px, kern_name), M, N, K, pad)
-    with open(os.path.join(px.LIB_DIR, KERNELS[kern_name]), "rb") as f:
+    with open(os.path.join(px.LIB_DIR, KERNELS[kern_name][0]), "rb") as f:
         mod = px.module_load_data(f.read())  # launched with the test's own grids
     for alpha, beta in ((1.0, 0.0), (0.75, -0.5)):
-        for entry, (tm, tn) in ENTRIES.items():
+        for entry, (tm, tn) in KERNELS[kern_name][1].items():
             fn = px.module_get_function(mod, entry)
             tiles = -(-M // tm) * -(-N // tn)
             outs = [case.launch(stream, fn, grid, 256, alpha, beta)
-                    for grid in {tiles, max(1, tiles // 2)}]
+                    for grid in (tiles, max(1, tiles // 2), min(8, tiles))]
             _check(case, outs[0], alpha, beta)
-            assert np.array_equal(outs[0], outs[-1]), entry
+            assert all(np.array_equal(outs[0], o) for o in outs), entry
     px.module_unload(mod)
 
 
 @pytest.mark.parametrize("kern_name", list(KERNELS))
 @pytest.mark.parametrize("M,N,K", [(64, 64, 4096), (65, 72, 2056), (200, 520, 3000),
-                                   (1000, 1000, 1000), (1208, 1208, 64), (300, 4096, 512)])
+                                   (1000, 1000, 1000), (1208, 1208, 64), (300, 4096, 512),
+                                   (2100, 2056, 40)])
 def test_rule_launches_meet_the_oracle(px_gpu, stream, kern_name, M, N, K):
     # through the built-in plan: the tile it picks, split over K into the
     # bound workspace where that is cheaper, and on a stream without one
