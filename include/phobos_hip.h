@@ -169,10 +169,11 @@ int phx_check_shape(phx_kernel k, const int64_t *dims, int ndims);
  * whose bound workspace holds at least *workspace_bytes: *splits K
  * chunks (gemm_fp32, gemm_fp16tc_fp32acc, gemm_fp16) or key chunks (flash),
  * 1 for none, and the workspace bytes that needs (0 for none).  With a
- * smaller workspace a launch takes fewer chunks, down to none.  For the
- * GEMMs it is the split of the 256 x 256 tile and the most a launch uses:
- * one that follows the built-in plan runs a smaller output tile instead, with
- * fewer chunks or none, where that is faster.  Other
+ * smaller workspace a launch takes fewer chunks, down to none.  It is the
+ * split of the 256 x 256 tile and of the regular flash kernel, and the most a
+ * launch uses: one that follows the built-in plan runs a smaller output tile
+ * or a small-launch flash kernel instead, with fewer chunks or none, where
+ * that is faster.  Other
  * kernels never split.  No counterpart in the reference, whose autotuner
  * picks tile sizes instead (phobos-bench/src/autotune.rs:98-192). */
 int phx_split_plan(phx_kernel k, const int64_t *dims, int ndims, int *splits,

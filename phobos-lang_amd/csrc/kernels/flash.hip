@@ -840,14 +840,32 @@ extern "C" __global__ __launch_bounds__(256) void flash_combine(const float *W, 
     for (int64_t i = (int64_t)phx_block_linear() * blockDim.x + threadIdx.x; i < total;
          i += (int64_t)phx_block_count() * blockDim.x) {
         const int64_t hqi = i / (D / 4), d4 = i % (D / 4);
-        float mx = ml[2 * hqi];
-        for (int32_t s = 1; s < nsplit; ++s) mx = fmaxf(mx, ml[2 * (s * nq + hqi)]);
-        float l = 0.0f;
+        // every chunk's m, l and sums are read in batches of four in flight (one
+        // at a time, 11 chunks waited for 22 memory latencies), merged in order
+        float mx = ml[2 * hqi], l = 0.0f;
         phx_f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int32_t s = 0; s < nsplit; ++s) {
-            const float w = __builtin_amdgcn_exp2f(ml[2 * (s * nq + hqi)] - mx);
-            l = l + w * ml[2 * (s * nq + hqi) + 1];
-            acc = acc + w * *(const phx_f4 *)(W + (s * nq + hqi) * D + 4 * d4);
+        for (int32_t s0 = 0; s0 < nsplit; s0 += 4) {
+            float2 v[4];
+            phx_f4 a[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int64_t r = (s0 + u < nsplit ? s0 + u : s0) * nq + hqi;
+                v[u] = *(const float2 *)(ml + 2 * r);
+                a[u] = *(const phx_f4 *)(W + r * D + 4 * d4);
+            }
+            float m4 = mx;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) m4 = fmaxf(m4, v[u].x);
+            const float c = __builtin_amdgcn_exp2f(mx - m4);  // 1 unless the max rose
+            l = l * c;
+            acc = acc * c;
+            mx = m4;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const float w = s0 + u < nsplit ? __builtin_amdgcn_exp2f(v[u].x - mx) : 0.0f;
+                l = l + w * v[u].y;
+                acc = acc + w * a[u];
+            }
         }
         const int64_t h = hqi / Nq, q = hqi % Nq;
         T *dst = O + h * ho + q * ldo + 4 * d4;
@@ -859,3 +877,6 @@ extern "C" __global__ __launch_bounds__(256) void flash_combine(const float *W, 
 #endif
     }
 }
+
+// ------------------------------------------------------ small launches
+#include "flash_w.h"

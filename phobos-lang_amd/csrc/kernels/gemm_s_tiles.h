@@ -138,9 +138,11 @@ __device__ __forceinline__ void s_body(const float *A, int64_t lda, const float 
         acc[0] = (phx_f16v){0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         acc[1] = acc[0];
 #pragma unroll
-        for (int p = 0; p < 2; ++p)
+        for (int p = 0; p < 2; ++p) {
 #pragma unroll
             for (int c = 0; c < DMA; ++c) copy(p, S[p], c);
+            __builtin_amdgcn_sched_barrier(0);  // the waits count on this order
+        }
         PHX_WAIT_VMCNT(DMA);
         __builtin_amdgcn_s_barrier();
         SFrags f[2];

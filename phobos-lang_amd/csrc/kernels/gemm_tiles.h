@@ -375,9 +375,11 @@ __device__ __forceinline__ void m_body(const TIn *A, const TIn *B, TO *C, uint32
         };
         constexpr int DMA = T::AC + T::BC;
 #pragma unroll
-        for (int p = 0; p < 3; ++p)
+        for (int p = 0; p < 3; ++p) {
 #pragma unroll
             for (int c = 0; c < DMA; ++c) copy(p, S[p], c);
+            __builtin_amdgcn_sched_barrier(0);  // the waits count on this order
+        }
         PHX_WAIT_VMCNT(2 * DMA);
         __builtin_amdgcn_s_barrier();
         MFrags<T> f[2];

@@ -688,25 +688,34 @@ static bool gemm_follows_rule(phx_kernel k, int64_t M, int64_t N, int64_t K) {
 // How many key chunks a flash launch is split into (1: no split).
 // PHX_FLASH_SPLIT=<n> in the environment forces n, for measurement.
 static bool flash_f16(phx_kernel k) { return k == PHX_FLASH_FP16 || k == PHX_FLASH_FP16_BH; }
-int flash_split(phx_kernel k, int64_t BH, int64_t Nq, int64_t Nk) {
+static int flash_split_rule(phx_kernel k, int64_t BH, int64_t Nq, int64_t Nk) {
     const int64_t qb = flash_f16(k) ? PHX_FA16_BR : PHX_FA_BR;
     const int64_t items = ((Nq + qb - 1) / qb) * BH;
     const int64_t nkb = (Nk + PHX_FA_BC - 1) / PHX_FA_BC;
-    int64_t sp;
-    phx_plan pin;
-    if (const char *env = getenv("PHX_FLASH_SPLIT")) {
-        sp = atoi(env);
-    } else if (pinned_plan(flash_key(k, BH, Nq, Nk), &pin)) {
-        sp = pin.splits;
-    } else {
-        if (2 * items >= PHX_FA_SLOTS) return 1;
-        const int64_t min_blocks =
-            flash_f16(k) ? PHX_FLASH_SPLIT_MIN_BLOCKS_F16 : PHX_FLASH_SPLIT_MIN_BLOCKS_F32;
-        sp = PHX_FLASH_SPLIT_TARGET / items;
-        if (sp > nkb / min_blocks) sp = nkb / min_blocks;
-        if (sp > PHX_SPLIT_MAX) sp = PHX_SPLIT_MAX;
-    }
+    if (2 * items >= PHX_FA_SLOTS) return 1;
+    const int64_t min_blocks =
+        flash_f16(k) ? PHX_FLASH_SPLIT_MIN_BLOCKS_F16 : PHX_FLASH_SPLIT_MIN_BLOCKS_F32;
+    int64_t sp = PHX_FLASH_SPLIT_TARGET / items;
+    if (sp > nkb / min_blocks) sp = nkb / min_blocks;
+    if (sp > PHX_SPLIT_MAX) sp = PHX_SPLIT_MAX;
     return round_split(nkb, sp);  // whole blocks per chunk; no empty chunk
+}
+
+int flash_split(phx_kernel k, int64_t BH, int64_t Nq, int64_t Nk) {
+    const int64_t nkb = (Nk + PHX_FA_BC - 1) / PHX_FA_BC;
+    phx_plan pin;
+    if (const char *env = getenv("PHX_FLASH_SPLIT")) return round_split(nkb, atoi(env));
+    if (pinned_plan(flash_key(k, BH, Nq, Nk), &pin)) return round_split(nkb, pin.splits);
+    return flash_split_rule(k, BH, Nq, Nk);
+}
+
+// Whether a flash launch follows the built-in plan, as gemm_follows_rule.
+static bool flash_follows_rule(phx_kernel k, int64_t BH, int64_t Nq, int64_t Nk) {
+    if (getenv("PHX_FLASH_SPLIT")) return false;
+    phx_plan pin;
+    if (!pinned_plan(flash_key(k, BH, Nq, Nk), &pin)) return true;
+    const int64_t nkb = (Nk + PHX_FA_BC - 1) / PHX_FA_BC;
+    return round_split(nkb, pin.splits) == flash_split_rule(k, BH, Nq, Nk);
 }
 
 // Bytes of partial results a split flash launch needs: per chunk and query,
@@ -721,6 +730,18 @@ size_t flash_split_bytes(int64_t BH, int64_t Nq, int sp) {
 int flash_split_functions(phx_kernel k, hipFunction_t *fs, hipFunction_t *fc) {
     if (int rc = aux_function(kSpecs[k].file, "flash_attention_split", fs)) return rc;
     return aux_function(kSpecs[k].file, "flash_combine", fc);
+}
+
+static int launch_flash_combine(hipFunction_t fc, uint64_t ws, int32_t nsplit, uint64_t o,
+                                int64_t BH, int64_t Nq, int64_t ldo, int64_t ho, hipStream_t s) {
+    void *ca[] = {&ws, &nsplit, &o, &BH, &Nq, &ldo, &ho};
+    const int64_t threads = BH * Nq * (PHX_FA_D / 4);
+    int64_t nb = (threads + PHX_REDUCE_THREADS - 1) / PHX_REDUCE_THREADS;
+    if (nb > 8192) nb = 8192;
+    hipError_t e = hipModuleLaunchKernel(fc, (uint32_t)nb, 1, 1, PHX_REDUCE_THREADS, 1, 1, 0, s, ca,
+                                         nullptr);
+    if (e != hipSuccess) return hip_error(e, "hipModuleLaunchKernel(flash_combine)");
+    return PHX_OK;
 }
 
 int launch_flash_split_ws(phx_kernel k, const Desc *t, int rank, int64_t BH, int64_t Nq,
@@ -741,14 +762,109 @@ int launch_flash_split_ws(phx_kernel k, const Desc *t, int rank, int64_t BH, int
     hipError_t e = hipModuleLaunchKernel(fs, (uint32_t)items, (uint32_t)sp, 1, kSpecs[k].block, 1,
                                          1, 0, s, sa, nullptr);
     if (e != hipSuccess) return hip_error(e, "hipModuleLaunchKernel(flash_attention_split)");
-    uint64_t o = t[3].ptr;
-    void *ca[] = {&ws, &nsplit, &o, &BH, &Nq, &ldo, &ho};
-    const int64_t threads = BH * Nq * (PHX_FA_D / 4);
-    int64_t nb = (threads + PHX_REDUCE_THREADS - 1) / PHX_REDUCE_THREADS;
-    if (nb > 8192) nb = 8192;
-    e = hipModuleLaunchKernel(fc, (uint32_t)nb, 1, 1, PHX_REDUCE_THREADS, 1, 1, 0, s, ca, nullptr);
-    if (e != hipSuccess) return hip_error(e, "hipModuleLaunchKernel(flash_combine)");
+    return launch_flash_combine(fc, ws, nsplit, t[3].ptr, BH, Nq, ldo, ho, s);
+}
+
+// The small-launch flash kernels (flash_w.h) and what they and the regular
+// one cost on MI355X in nanoseconds: a workgroup takes `q` queries and walks
+// its key chunk `keys` keys a step, shared by `kg` key groups of its waves;
+// `step` for one workgroup per CU, `pair` for two sharing one (0: only one
+// fits).  A split adds its merge: 2.3 us and the partial results, 264 bytes
+// per query and chunk, at 2.3 TB/s.  Fitted to HIP event times at 16 shapes
+// of each precision (within 8%); f16, one head of 4096^2: the wide kernel in
+// 4 chunks 14.6 us against 23.2 for the regular one in 11; 16 heads of 1000^2
+// 10.5 against 20.4; 8 heads of 512^2: 7.1 (narrow) against 13.2; 16 heads of
+// 4096^2: the regular one 84 against about 100.  f32: 4 heads of 1000 x 4133
+// the wide kernel in 2 chunks 42.7 against 51, 16 heads of 200 x 300 11.3
+// (narrow) against 20.2.
+struct FTile {
+    const char *entry;  // null: the regular kernel
+    int64_t q, keys, kg;
+    uint32_t threads;
+    int64_t fixed, step, pair, round;
+};
+static const FTile kFlash16[] = {
+    {nullptr, 256, 64, 1, PHX_FA16_THREADS, 5700, 1100, 2270, 1500},
+    {"flash_w4", 32, 64, 4, 256, 5000, 1080, 2450, 2500},
+    {"flash_w2x4", 64, 64, 4, 512, 5000, 1380, 0, 3000},
+};
+static const FTile kFlash32[] = {
+    {nullptr, 128, 64, 1, PHX_FA_THREADS, 4200, 4340, 8200, 1500},
+    {"flash_w4", 32, 32, 4, 256, 5000, 2270, 4100, 2500},
+    {"flash_w8", 32, 32, 8, 512, 5200, 4050, 0, 2500},
+};
+
+static int64_t ftile_cost(const FTile &f, int64_t BH, int64_t Nq, int64_t Nk, int sp) {
+    const int64_t nkb = (Nk + PHX_FA_BC - 1) / PHX_FA_BC;
+    const int64_t chunk = (nkb + sp - 1) / sp * PHX_FA_BC;
+    const int64_t keys = chunk < Nk ? chunk : Nk;
+    const int64_t steps = ((keys + f.keys - 1) / f.keys + f.kg - 1) / f.kg;
+    const int64_t n = ((Nq + f.q - 1) / f.q * BH * sp + 255) / 256;
+    int64_t ns = f.fixed;
+    if (n == 1) {
+        ns += steps * f.step;
+    } else {
+        const int64_t rounds = f.pair ? (n + 1) / 2 : n;
+        ns += rounds * steps * (f.pair ? f.pair : f.step) + (rounds - 1) * f.round;
+    }
+    if (sp > 1) ns += 2300 + sp * BH * Nq * 264 / 2300;
+    return ns;
+}
+
+int flash_small_functions(phx_kernel k) {
+    const FTile *tiles = flash_f16(k) ? kFlash16 : kFlash32;
+    hipFunction_t f;
+    for (int i = 1; i < 3; ++i)
+        if (int rc = aux_function(kSpecs[k].file, tiles[i].entry, &f)) return rc;
     return PHX_OK;
+}
+
+// Launches a flash problem that follows the built-in plan on a small-launch
+// kernel, in at most max_sp key chunks (whose partial results go to ws), when
+// that is estimated faster than the regular kernel in max_sp chunks; else
+// leaves *done false.
+int launch_flash_small(phx_kernel k, const Desc *t, int rank, int64_t BH, int64_t Nq, int64_t Nk,
+                       float scale, int max_sp, hipStream_t s, uint64_t ws, bool *done) {
+    *done = false;
+    if (!flash_follows_rule(k, BH, Nq, Nk)) return PHX_OK;
+    const int r = rank - 2;  // index of the row stride
+    // row strides the kernels' 32-bit offsets take (as the regular entries check)
+    for (int i = 0; i < 4; ++i)
+        if (t[i].stride[r] < PHX_FA_D || (i == 0 || i == 3 ? Nq : Nk) * t[i].stride[r] * 4 > INT32_MAX)
+            return PHX_OK;
+    const FTile *tiles = flash_f16(k) ? kFlash16 : kFlash32;
+    const int64_t nkb = (Nk + PHX_FA_BC - 1) / PHX_FA_BC;
+    const FTile *best = nullptr;
+    int64_t least = ftile_cost(tiles[0], BH, Nq, Nk, max_sp);
+    int32_t sp = 1;
+    for (int i = 1; i < 3; ++i)
+        for (int want = 1; want <= max_sp; ++want) {
+            const int c = round_split(nkb, want);
+            const int64_t ns = ftile_cost(tiles[i], BH, Nq, Nk, c);
+            if (ns < least) {
+                best = &tiles[i];
+                least = ns;
+                sp = c;
+            }
+        }
+    if (!best) return PHX_OK;
+    hipFunction_t f, fc = nullptr;
+    if (int rc = aux_function(kSpecs[k].file, best->entry, &f)) return rc;
+    if (sp > 1)
+        if (int rc = aux_function(kSpecs[k].file, "flash_combine", &fc)) return rc;
+    uint64_t q = t[0].ptr, kk = t[1].ptr, v = t[2].ptr, o = t[3].ptr;
+    int64_t ldq = t[0].stride[r], ldk = t[1].stride[r], ldv = t[2].stride[r], ldo = t[3].stride[r];
+    int64_t hq = r ? t[0].stride[0] : 0, hk = r ? t[1].stride[0] : 0, hv = r ? t[2].stride[0] : 0;
+    int64_t ho = r ? t[3].stride[0] : 0;
+    int64_t kchunk = (nkb + sp - 1) / sp * PHX_FA_BC;
+    void *a[] = {&q,   &kk,  &v,  &o,  &ws, &BH, &Nq,     &Nk, &ldq, &ldk,
+                 &ldv, &ldo, &hq, &hk, &hv, &ho, &kchunk, &sp, &scale};
+    const int64_t items = (Nq + best->q - 1) / best->q * BH;
+    hipError_t e = hipModuleLaunchKernel(f, (uint32_t)items, (uint32_t)sp, 1, best->threads, 1, 1, 0,
+                                         s, a, nullptr);
+    if (e != hipSuccess) return hip_error(e, "hipModuleLaunchKernel(flash_w)");
+    *done = true;
+    return sp > 1 ? launch_flash_combine(fc, ws, sp, o, BH, Nq, ldo, ho, s) : PHX_OK;
 }
 
 static int flash_split_fit(phx_kernel k, int64_t BH, int64_t Nq, int64_t Nk, size_t cap) {
@@ -868,9 +984,14 @@ int launch_raw(hipFunction_t f, const uint32_t grid[3], const uint32_t block[3],
             const int64_t BH = bh ? d[0] : 1, Nq = d[bh], Nk = d[bh + 1];
             const Workspace w = stream_workspace(s);
             const int sp = flash_split_fit((phx_kernel)k, BH, Nq, Nk, w.bytes);
+            float scale;  // the f32 scalar after the four memrefs
+            memcpy(&scale, args[bh ? 36 : 28], 4);
+            bool done = false;
+            if (int rc = launch_flash_small((phx_kernel)k, t, bh ? 3 : 2, BH, Nq, Nk, scale, sp, s,
+                                            w.ptr, &done))
+                return rc;
+            if (done) return PHX_OK;
             if (sp > 1) {
-                float scale;  // the f32 scalar after the four memrefs
-                memcpy(&scale, args[bh ? 36 : 28], 4);
                 hipFunction_t fs, fc;
                 if (int rc = flash_split_functions((phx_kernel)k, &fs, &fc)) return rc;
                 return launch_flash_split_ws((phx_kernel)k, t, bh ? 3 : 2, BH, Nq, Nk, scale, sp,

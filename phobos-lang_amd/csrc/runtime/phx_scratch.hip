@@ -47,7 +47,8 @@ int scratch_setup(int device) {
     g_missing.clear();
     for (int i = 0; i < 2; ++i) {
         if (builtin(bh[i], &g_bh[i]) ||
-            flash_split_functions(bh[i], &g_split[i], &g_combine[i])) {
+            flash_split_functions(bh[i], &g_split[i], &g_combine[i]) ||
+            flash_small_functions(bh[i])) {
             g_bh[i] = g_split[i] = g_combine[i] = nullptr;
             g_missing = phx_last_error();  // the other entry points report it on use
         }
@@ -91,28 +92,32 @@ extern "C" int phx_flash_attention_bh_noalloc(phx_stream s, phx_kernel k, uint64
                              "%u (phx_flash_attention_bh takes any size)",
                              (long long)BH, (long long)Nq, (long long)Nk, sp, need,
                              (unsigned)PHX_SCRATCH_BYTES);
-        Desc t[4];
-        const uint64_t ptr[4] = {q, kk, v, o};
-        const int64_t n[4] = {Nq, Nk, Nk, Nq};
-        for (int j = 0; j < 4; ++j) {
-            t[j].ptr = ptr[j];
-            t[j].size[0] = BH;
-            t[j].size[1] = n[j];
-            t[j].size[2] = D;
-            t[j].stride[0] = n[j] * D;
-            t[j].stride[1] = D;
-            t[j].stride[2] = 1;
-        }
+    }
+    Desc t[4];
+    const uint64_t ptr[4] = {q, kk, v, o};
+    const int64_t n[4] = {Nq, Nk, Nk, Nq};
+    for (int j = 0; j < 4; ++j) {
+        t[j].ptr = ptr[j];
+        t[j].size[0] = BH;
+        t[j].size[1] = n[j];
+        t[j].size[2] = D;
+        t[j].stride[0] = n[j] * D;
+        t[j].stride[1] = D;
+        t[j].stride[2] = 1;
+    }
+    bool done = false;
+    if (int rc = launch_flash_small(k, t, 3, BH, Nq, Nk, scale, sp, (hipStream_t)s, g_scratch[dev],
+                                    &done))
+        return rc;
+    if (done) return PHX_OK;
+    if (sp > 1)
         return launch_flash_split_ws(k, t, 3, BH, Nq, Nk, scale, sp, (hipStream_t)s,
                                      g_scratch[dev], g_split[i], g_combine[i]);
-    }
     // no split: the batched kernel itself, with the exploded-memref argument
     // list built on the stack
     uint64_t slots[37];
     void *args[37];
     int a = 0;
-    const uint64_t ptr[4] = {q, kk, v, o};
-    const int64_t n[4] = {Nq, Nk, Nk, Nq};
     for (int j = 0; j < 4; ++j) {
         const int64_t vals[9] = {0, 0, 0, BH, n[j], D, n[j] * D, D, 1};
         for (int r = 0; r < 9; ++r) {
