@@ -33,6 +33,7 @@ int launch_flash_split_ws(phx_kernel k, const Desc *t, int rank, int64_t BH, int
 // the small-launch kernels (phx_runtime.cpp): whether the launch took one of
 // them is left in *done
 int flash_small_functions(phx_kernel k);
+bool flash_follows_rule(phx_kernel k, int64_t BH, int64_t Nq, int64_t Nk);
 int launch_flash_small(phx_kernel k, const Desc *t, int rank, int64_t BH, int64_t Nq, int64_t Nk,
                        float scale, int max_sp, hipStream_t s, uint64_t ws, bool *done);
 // the allocation-free entry point's per-device set-up (phx_scratch.hip)

@@ -12,7 +12,6 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
-#include <deque>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -71,6 +70,7 @@ struct State {
     std::unordered_map<hipModule_t, std::string> module_files;  // module -> file name
     std::unordered_map<hipFunction_t, std::pair<int, hipModule_t>> aliases;
     std::unordered_map<std::string, hipFunction_t> aux;  // "file:entry" -> function
+    std::atomic<uint64_t> epoch{1};  // of the loaded modules; phx_shutdown begins the next
     std::mutex mu;
 };
 static State g;
@@ -136,11 +136,34 @@ int builtin(phx_kernel k, hipFunction_t *out) {
     return PHX_OK;
 }
 
+static int find_aux(const char *file, const char *entry, hipFunction_t *out);
+
 // Entry points of the built-in code objects that no .ph kernel names (the
 // split-K and split-key kernels the runtime launches itself), by file and
 // entry name; loaded on first use.
 int aux_function(const char *file, const char *entry, hipFunction_t *out) {
     if (int rc = ensure_init()) return rc;
+    // The names are string literals, so each thread remembers its last few by
+    // address (the locked map lookup and its key cost a launch 0.15 us); an
+    // answer is good until the modules it came from are unloaded.
+    struct Known {
+        const char *file = nullptr, *entry = nullptr;
+        uint64_t epoch = 0;
+        hipFunction_t f = nullptr;
+    };
+    static thread_local Known known[32];
+    Known &kn = known[(((uintptr_t)entry >> 2) ^ ((uintptr_t)file >> 5)) % 32];
+    const uint64_t epoch = g.epoch.load(std::memory_order_acquire);
+    if (kn.file == file && kn.entry == entry && kn.epoch == epoch) {
+        *out = kn.f;
+        return PHX_OK;
+    }
+    if (int rc = find_aux(file, entry, out)) return rc;
+    kn = Known{file, entry, epoch, *out};
+    return PHX_OK;
+}
+
+static int find_aux(const char *file, const char *entry, hipFunction_t *out) {
     std::lock_guard<std::mutex> lock(g.mu);
     const std::string key = std::string(file) + ":" + entry;
     auto fit = g.aux.find(key);
@@ -172,14 +195,30 @@ int aux_function(const char *file, const char *entry, hipFunction_t *out) {
 
 // ------------------------------------------------------------------ args
 // Holds the values of an exploded-memref argument list at stable addresses
-// plus the void* array hipModuleLaunchKernel reads.
+// plus the void* array hipModuleLaunchKernel reads: on the stack up to the 48
+// words every built-in needs, on the heap beyond (a COMPUTE of many tiles).
 struct ArgPack {
-    std::deque<uint64_t> slots;  // deque: push_back keeps earlier addresses valid
-    std::vector<void *> ptrs;
-    explicit ArgPack(size_t cap) { ptrs.reserve(cap); }
+    static constexpr size_t kInline = 48;
+    uint64_t words[kInline];
+    void *inline_ptrs[kInline];
+    std::vector<uint64_t> more_words;
+    std::vector<void *> more_ptrs;
+    uint64_t *slots = words;
+    void **ptrs = inline_ptrs;
+    size_t n = 0;
+    explicit ArgPack(size_t cap) {
+        if (cap <= kInline) return;
+        more_words.resize(cap);
+        more_ptrs.resize(cap);
+        slots = more_words.data();
+        ptrs = more_ptrs.data();
+    }
+    ArgPack(const ArgPack &) = delete;
+    ArgPack &operator=(const ArgPack &) = delete;
     void push_bits(uint64_t v) {
-        slots.push_back(v);
-        ptrs.push_back(&slots.back());
+        slots[n] = v;
+        ptrs[n] = &slots[n];
+        ++n;
     }
     void ptr(uint64_t p) { push_bits(p); }
     void idx(int64_t v, int bits) {
@@ -354,8 +393,10 @@ struct PlanKeyHash {
 };
 std::mutex g_plan_mu;
 std::unordered_map<PlanKey, phx_plan, PlanKeyHash> g_plans;
+std::atomic<size_t> g_num_plans{0};  // g_plans.size(), read without the lock
 
 bool pinned_plan(const PlanKey &key, phx_plan *out) {  // out may be null
+    if (g_num_plans.load(std::memory_order_acquire) == 0) return false;
     std::lock_guard<std::mutex> lock(g_plan_mu);
     auto it = g_plans.find(key);
     if (it == g_plans.end()) return false;
@@ -545,10 +586,9 @@ static int launch_gemm_split_ws(phx_kernel k, const char *entry, int64_t tm, int
     return PHX_OK;
 }
 
-// The split count a GEMM launch on a stream whose workspace holds cap bytes
-// runs with: gemm_split's plan, cut to what fits.
-static int gemm_split_fit(phx_kernel k, int64_t M, int64_t N, int64_t K, size_t cap) {
-    const int sp = gemm_split(k, M, N, K);
+// The split count a GEMM launch planned for sp chunks runs with on a stream
+// whose workspace holds cap bytes: the most that fit.
+static int gemm_split_fit(int sp, int64_t M, int64_t N, int64_t K, size_t cap) {
     if (sp < 2) return 1;
     const int64_t steps = (K + PHX_SPLIT_KSTEP - 1) / PHX_SPLIT_KSTEP;
     return fit_split(steps, sp, gemm_split_bytes(M, N, 1), cap);
@@ -609,8 +649,10 @@ static const HTile *gemm_tile_plan(phx_kernel k, int64_t M, int64_t N, int64_t K
     const HTile *best = nullptr;
     int64_t least = 0;
     for (int i = 0; i < kHTiles; ++i)
-        for (int want = 1; want <= max_sp; ++want) {
-            const int sp = round_split(units, want);
+        for (int want = 1, last = 0; want <= max_sp; ++want) {
+            const int sp = want == 1 ? 1 : round_split(units, want);
+            if (sp == last) continue;
+            last = sp;
             const int64_t ns = htile_cost(tiles[i], M, N, K, sp);
             if (!best || ns < least) {
                 best = &tiles[i];
@@ -661,8 +703,10 @@ static const SHTile *s_tile_plan(int64_t M, int64_t N, int64_t K, int max_sp, in
     const SHTile *best = nullptr;
     int64_t least = 0;
     for (const SHTile &ti : kSTiles)
-        for (int want = 1; want <= max_sp; ++want) {
-            const int sp = round_split(units, want);
+        for (int want = 1, last = 0; want <= max_sp; ++want) {
+            const int sp = want == 1 ? 1 : round_split(units, want);
+            if (sp == last) continue;
+            last = sp;
             const int64_t ns = stile_cost(ti, M, N, K, sp);
             if (!best || ns < least) {
                 best = &ti;
@@ -710,7 +754,7 @@ int flash_split(phx_kernel k, int64_t BH, int64_t Nq, int64_t Nk) {
 }
 
 // Whether a flash launch follows the built-in plan, as gemm_follows_rule.
-static bool flash_follows_rule(phx_kernel k, int64_t BH, int64_t Nq, int64_t Nk) {
+bool flash_follows_rule(phx_kernel k, int64_t BH, int64_t Nq, int64_t Nk) {
     if (getenv("PHX_FLASH_SPLIT")) return false;
     phx_plan pin;
     if (!pinned_plan(flash_key(k, BH, Nq, Nk), &pin)) return true;
@@ -819,14 +863,13 @@ int flash_small_functions(phx_kernel k) {
     return PHX_OK;
 }
 
-// Launches a flash problem that follows the built-in plan on a small-launch
+// Launches a flash problem (one that follows the built-in plan) on a small-launch
 // kernel, in at most max_sp key chunks (whose partial results go to ws), when
 // that is estimated faster than the regular kernel in max_sp chunks; else
 // leaves *done false.
 int launch_flash_small(phx_kernel k, const Desc *t, int rank, int64_t BH, int64_t Nq, int64_t Nk,
                        float scale, int max_sp, hipStream_t s, uint64_t ws, bool *done) {
     *done = false;
-    if (!flash_follows_rule(k, BH, Nq, Nk)) return PHX_OK;
     const int r = rank - 2;  // index of the row stride
     // row strides the kernels' 32-bit offsets take (as the regular entries check)
     for (int i = 0; i < 4; ++i)
@@ -838,8 +881,10 @@ int launch_flash_small(phx_kernel k, const Desc *t, int rank, int64_t BH, int64_
     int64_t least = ftile_cost(tiles[0], BH, Nq, Nk, max_sp);
     int32_t sp = 1;
     for (int i = 1; i < 3; ++i)
-        for (int want = 1; want <= max_sp; ++want) {
-            const int c = round_split(nkb, want);
+        for (int want = 1, last = 0; want <= max_sp; ++want) {
+            const int c = want == 1 ? 1 : round_split(nkb, want);
+            if (c == last) continue;
+            last = c;
             const int64_t ns = ftile_cost(tiles[i], BH, Nq, Nk, c);
             if (ns < least) {
                 best = &tiles[i];
@@ -867,8 +912,7 @@ int launch_flash_small(phx_kernel k, const Desc *t, int rank, int64_t BH, int64_
     return sp > 1 ? launch_flash_combine(fc, ws, sp, o, BH, Nq, ldo, ho, s) : PHX_OK;
 }
 
-static int flash_split_fit(phx_kernel k, int64_t BH, int64_t Nq, int64_t Nk, size_t cap) {
-    const int sp = flash_split(k, BH, Nq, Nk);
+static int flash_split_fit(int sp, int64_t BH, int64_t Nq, int64_t Nk, size_t cap) {
     if (sp < 2) return 1;
     const int64_t nkb = (Nk + PHX_FA_BC - 1) / PHX_FA_BC;
     return fit_split(nkb, sp, flash_split_bytes(BH, Nq, 1), cap);
@@ -913,11 +957,14 @@ int launch_raw(hipFunction_t f, const uint32_t grid[3], const uint32_t block[3],
         if (k == PHX_GEMM_FP32 || k == PHX_GEMM_FP16TC_FP32ACC || k == PHX_GEMM_FP16) {
             if (int rc = check_shape((phx_kernel)k, d, nd)) return rc;
             const Workspace w = stream_workspace(s);
-            const int sp = gemm_split_fit((phx_kernel)k, d[0], d[1], d[2], w.bytes);
+            const bool rule = gemm_follows_rule((phx_kernel)k, d[0], d[1], d[2]);
+            const int planned = rule ? gemm_split_rule((phx_kernel)k, d[0], d[1], d[2])
+                                     : gemm_split((phx_kernel)k, d[0], d[1], d[2]);
+            const int sp = gemm_split_fit(planned, d[0], d[1], d[2], w.bytes);
             float alpha, beta;  // the two f32 scalars after the three memrefs
             memcpy(&alpha, args[21], 4);
             memcpy(&beta, args[22], 4);
-            if (gemm_follows_rule((phx_kernel)k, d[0], d[1], d[2]) && dense_rows(t, d)) {
+            if (rule && dense_rows(t, d)) {
                 int msp = 1;
                 const char *entry, *split_entry;
                 int64_t tm, tn;
@@ -983,13 +1030,17 @@ int launch_raw(hipFunction_t f, const uint32_t grid[3], const uint32_t block[3],
             const bool bh = nd == 4;
             const int64_t BH = bh ? d[0] : 1, Nq = d[bh], Nk = d[bh + 1];
             const Workspace w = stream_workspace(s);
-            const int sp = flash_split_fit((phx_kernel)k, BH, Nq, Nk, w.bytes);
+            const bool rule = flash_follows_rule((phx_kernel)k, BH, Nq, Nk);
+            const int planned = rule ? flash_split_rule((phx_kernel)k, BH, Nq, Nk)
+                                     : flash_split((phx_kernel)k, BH, Nq, Nk);
+            const int sp = flash_split_fit(planned, BH, Nq, Nk, w.bytes);
             float scale;  // the f32 scalar after the four memrefs
             memcpy(&scale, args[bh ? 36 : 28], 4);
             bool done = false;
-            if (int rc = launch_flash_small((phx_kernel)k, t, bh ? 3 : 2, BH, Nq, Nk, scale, sp, s,
-                                            w.ptr, &done))
-                return rc;
+            if (rule)
+                if (int rc = launch_flash_small((phx_kernel)k, t, bh ? 3 : 2, BH, Nq, Nk, scale, sp,
+                                                s, w.ptr, &done))
+                    return rc;
             if (done) return PHX_OK;
             if (sp > 1) {
                 hipFunction_t fs, fc;
@@ -1176,6 +1227,7 @@ int phx_shutdown(void) {
         g_ws.clear();
     }
     std::lock_guard<std::mutex> lock(g.mu);
+    g.epoch.fetch_add(1, std::memory_order_acq_rel);
     for (auto &kv : g.modules) (void)hipModuleUnload(kv.second);
     g.modules.clear();
     for (auto &f : g.fns) f.store(nullptr, std::memory_order_release);
@@ -1477,12 +1529,14 @@ int phx_plan_pin(phx_kernel k, const int64_t *dims, int ndims, const phx_plan *p
         g_plans[key] = *plan;
     else
         g_plans.erase(key);
+    g_num_plans.store(g_plans.size(), std::memory_order_release);
     return PHX_OK;
 }
 
 int phx_plan_unpin_all(void) {
     std::lock_guard<std::mutex> lock(g_plan_mu);
     g_plans.clear();
+    g_num_plans.store(0, std::memory_order_release);
     return PHX_OK;
 }
 
@@ -1517,7 +1571,7 @@ int phx_compute(phx_function f, int bits, const phx_tile_arg *tiles, uint32_t nt
         pack.memref(t.addr, shape, (int)t.rank, bits);
     }
     if (next_tile != ntiles) return set_error(PHX_E_INVALID, "%u tiles left unplaced", ntiles - next_tile);
-    return launch_raw((hipFunction_t)f, grid, cta, 0, (hipStream_t)s, pack.ptrs.data());
+    return launch_raw((hipFunction_t)f, grid, cta, 0, (hipStream_t)s, pack.ptrs);
 }
 
 // ------------------------------------------------------------------ typed launches
@@ -1525,9 +1579,9 @@ static int launch_builtin(phx_kernel k, const int64_t *dims, int nd, ArgPack &pa
                           hipStream_t s) {
     hipFunction_t f;
     if (int rc = builtin(k, &f)) return rc;
-    uint32_t grid[3], block[3];
-    if (int rc = grid_for(k, dims, nd, grid, block)) return rc;
-    return launch_raw(f, grid, block, 0, s, pack.ptrs.data());
+    if (int rc = check_shape(k, dims, nd)) return rc;
+    const uint32_t one[3] = {1, 1, 1};  // replaced by the built-in's own geometry
+    return launch_raw(f, one, one, 0, s, pack.ptrs);
 }
 
 int phx_saxpy(phx_stream s, uint64_t x, uint64_t y, uint64_t out, int64_t n, float alpha) {

@@ -106,9 +106,10 @@ extern "C" int phx_flash_attention_bh_noalloc(phx_stream s, phx_kernel k, uint64
         t[j].stride[2] = 1;
     }
     bool done = false;
-    if (int rc = launch_flash_small(k, t, 3, BH, Nq, Nk, scale, sp, (hipStream_t)s, g_scratch[dev],
-                                    &done))
-        return rc;
+    if (flash_follows_rule(k, BH, Nq, Nk))
+        if (int rc = launch_flash_small(k, t, 3, BH, Nq, Nk, scale, sp, (hipStream_t)s,
+                                        g_scratch[dev], &done))
+            return rc;
     if (done) return PHX_OK;
     if (sp > 1)
         return launch_flash_split_ws(k, t, 3, BH, Nq, Nk, scale, sp, (hipStream_t)s,

@@ -350,6 +350,8 @@ def _addr(buf, nbytes, what):
     """Device address of `buf` (a DeviceBuffer or a raw address).  For a
     DeviceBuffer the size is checked against the bytes the kernel touches, so
     a wrong buffer raises on the host instead of faulting the GPU."""
+    if type(buf) is int:
+        return buf
     if isinstance(buf, DeviceBuffer):
         if buf.nbytes < nbytes:
             raise PhxError(PHX_E_INVALID, f"{what}: buffer holds {buf.nbytes} B, kernel "
