@@ -1063,13 +1063,13 @@ extern "C" __global__ __launch_bounds__(W8_NT, 1) void gemm_w8_splitk(const TIn 
 // ------------------------------------------------------ smaller tiles
 #include "gemm_tiles.h"
 #ifdef PHX_GEMM_TC
-typedef MTile<64, 64, 64, 2, 4, 2> M64;
-typedef MTile<128, 64, 64, 1, 4, 1> M128x64;
-typedef MTile<128, 128, 32, 1, 2, 2> M128;
+typedef MTile<64, 64, 64, 4, 2> M64;
+typedef MTile<128, 64, 64, 4, 1> M128x64;
+typedef MTile<128, 128, 32, 2, 2> M128;
 #else
-typedef MTile<64, 64, 64, 0, 4, 2> M64;
-typedef MTile<128, 64, 64, 0, 2, 1> M128x64;
-typedef MTile<128, 128, 64, 0, 1, 1> M128;
+typedef MTile<64, 64, 64, 4, 2> M64;
+typedef MTile<128, 64, 64, 2, 1> M128x64;
+typedef MTile<128, 128, 64, 1, 1> M128;
 #endif
 GEMM_M(m64, M64)
 GEMM_M(m128x64, M128x64)

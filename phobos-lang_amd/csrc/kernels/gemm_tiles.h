@@ -16,8 +16,8 @@
 // with its best split): gemm_fp16 512^3 4.8 (64 x 64) against 14.0, 1024^3
 // 7.0 (64 x 64) against 22.8, 1280^3 10.6 (128 x 64) against 22.4, 2048^3
 // 21.7 (128 x 128) against 36.3, 2560^3 44.3 (128 x 128) against 53.1;
-// gemm_fp16tc_fp32acc 512^3 6.7 against 14.4, 1024^3 10.8 against 21.0,
-// 2048^3 33.2 against 40.3.  At 3072^3 the 256 x 256 tile is the faster one
+// gemm_fp16tc_fp32acc 512^3 6.0 against 14.5, 1024^3 10.1 against 20.9,
+// 2048^3 30.0 against 39.8.  At 3072^3 the 256 x 256 tile is the faster one
 // (64.4 against 75.9).
 //
 // Design: 4 waves in a 2 x 2 arrangement; v_mfma_f32_32x32x16_f16; each k
@@ -26,7 +26,7 @@
 // last slice, so the next step's first operands are read while the last
 // slice multiplies.  gemm_fp16 copies global -> LDS into 4 stages, three
 // steps ahead; gemm_fp16tc converts step k + 2 into a 3-stage ring from
-// registers loaded NS steps before.  The k slices add into AS accumulator
+// registers loaded one step before.  The k slices add into AS accumulator
 // sets in turn, summed pairwise at the end: the f32 rounding of a short chain
 // without a split (gemm_fp16tc at 1024^3, against f64: 1.0e-7 with four sets
 // on the 64 x 64 tile, 1.8e-7 with one, 1.1e-7 for the 4-way split it
@@ -36,10 +36,9 @@
 #include <type_traits>
 
 // A TM x TN output tile per workgroup, K steps of TK.
-template <int TM_, int TN_, int TK_, int NS_, int AS_, int OCC_>
+template <int TM_, int TN_, int TK_, int AS_, int OCC_>
 struct MTile {
     static constexpr int TM = TM_, TN = TN_, TK = TK_;
-    static constexpr int NS = NS_;    // tc: register sets of loads in flight
     static constexpr int AS = AS_;    // accumulator sets: k slice s adds into set s % AS
     static constexpr int OCC = OCC_;  // waves per SIMD the registers must allow
     static constexpr int WMT = TM / 2, WNT = TN / 2;
@@ -284,12 +283,12 @@ __device__ __forceinline__ void m_body(const TIn *A, const TIn *B, TO *C, uint32
             *(phx_u4 *)(st + T::ABYTES +
                         mb_off<T>(i * (NT / T::CPB) + tid / T::CPB, tid % T::CPB)) = pack(c);
         };
-        MRegs<T> R[T::NS];
+        MRegs<T> R;
         {
             MRegs<T> P[2];
 #pragma unroll
-            for (int p = 0; p < 2 + T::NS; ++p) {
-                MRegs<T> &d = p < 2 ? P[p] : R[p % T::NS];
+            for (int p = 0; p < 3; ++p) {
+                MRegs<T> &d = p < 2 ? P[p] : R;
 #pragma unroll
                 for (int i = 0; i < T::AC; ++i) load_a(d.a[i], p, i);
 #pragma unroll
@@ -308,38 +307,35 @@ __device__ __forceinline__ void m_body(const TIn *A, const TIn *B, TO *C, uint32
         MFrags<T> f[2];
 #pragma unroll
         for (int r = 0; r < T::MI + T::NJ; ++r) m_read<T>(f[0], lds, 0, wm, wn, lane, r);
-        // step k: its data in stage c0, step k+1's in c1; step k+2's is
-        // converted into c2, which every wave has left since step k-1's barrier
-        uint32_t c0 = 0, c1 = T::STAGE, c2 = 2 * T::STAGE;
+        // step k = u mod 3: its data in stage u, step k+1's in the next; step
+        // k+2's is converted into the third, which every wave has left since
+        // step k-1's barrier.  Whole rings, so that every stage's address is
+        // an immediate (a rotating base cost the 128 x 128 tile 8%).
         auto step = [&](uint32_t k, int u) {
-            MRegs<T> &d = R[u % T::NS];
+            char *const fill = lds + (u + 2) % 3 * T::STAGE;
             m_step<T, T::AC + T::BC>(
-                acc, f, lds + c0, lds + c1, wm, wn, lane,
+                acc, f, lds + u * T::STAGE, lds + (u + 1) % 3 * T::STAGE, wm, wn, lane,
                 [&](int c) {
                     if (c < T::AC) {
-                        store_a(d.a[c], lds + c2, c);
-                        load_a(d.a[c], k + 2 + T::NS, c);
+                        store_a(R.a[c], fill, c);
+                        load_a(R.a[c], k + 3, c);
                     } else {
-                        store_b(d.b[c - T::AC], lds + c2, c - T::AC);
-                        load_b(d.b[c - T::AC], k + 2 + T::NS, c - T::AC);
+                        store_b(R.b[c - T::AC], fill, c - T::AC);
+                        load_b(R.b[c - T::AC], k + 3, c - T::AC);
                     }
                 },
                 [&] {
                     PHX_WAIT_VM_LGKM0(63);
                     __builtin_amdgcn_s_barrier();
                 });
-            const uint32_t t3 = c0;
-            c0 = c1;
-            c1 = c2;
-            c2 = t3;
         };
         uint32_t kt = 0;
-        for (; kt + T::NS <= nk; kt += T::NS) {
+        for (; kt + 3 <= nk; kt += 3) {
 #pragma unroll
-            for (int u = 0; u < T::NS; ++u) step(kt + u, u);
+            for (int u = 0; u < 3; ++u) step(kt + u, u);
         }
 #pragma unroll
-        for (int u = 0; u < T::NS - 1; ++u)
+        for (int u = 0; u < 2; ++u)
             if (kt + u < nk) step(kt + u, u);
         PHX_WAIT_VMCNT(0);
         __syncthreads();

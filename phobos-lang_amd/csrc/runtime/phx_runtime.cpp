@@ -598,28 +598,30 @@ static int gemm_split_fit(int sp, int64_t M, int64_t N, int64_t K, size_t cap) {
 // chooses among, and what one costs on MI355X, in nanoseconds.  A launch of
 // tiles x splits workgroups runs ceil(workgroups / 256) rounds on the CUs: a
 // single round takes `round` plus `step` per 64 columns of its K chunk, of
-// which `idle` percent are left when few CUs are busy (less contention and,
-// for the big tiles, a higher clock); each of several rounds takes `round2`
-// plus `step2` (co-resident workgroups overlap).  Fitted to HIP event times
-// over K = 64 .. 4096 and 64^2 .. 4096^2 outputs, where the pick was the
-// fastest tile or within 10% of it: 1024^2 outputs 64 x 64 (gemm_fp16 at K
-// 1024 7.0 us against 22.8 for the 256 x 256 tile split 4 ways), 1280^2 128 x
-// 64 (10.6 against 22.4), 2048^2 128 x 128 (21.7 against 36.3), 3072^2 256 x
-// 256 (64.4 against 75.9).
+// which `idle` percent are left when few CUs are busy (less contention, fewer
+// bytes of C and, for the big tiles, a higher clock); each of several rounds
+// takes `round2` plus `step2` (co-resident workgroups overlap).  Fitted to HIP
+// event times over K = 64 .. 4096 and 64^2 .. 4096^2 outputs, where the pick
+// was the fastest tile or within 10% of it, and within 3% of the 256 x 256
+// tile (gemm_fp16tc 4056 x 2104 x 192: 14.9 us for it, 17.2 for 128 x 128;
+// 2816 x 2816 x 2048: 53.4, 54.9 for the pick, 128 x 128): 1024^2 outputs 64 x
+// 64 (gemm_fp16 at K 1024 7.0 us against 22.8 for the 256 x 256 tile split 4
+// ways), 1280^2 128 x 64 (10.5 against 22.0), 2048^2 128 x 128 (21.7 against
+// 36.3), 3072^2 256 x 256 (60.5 against 69.0).
 struct HTile {
     const char *entry, *split_entry;
     int64_t tm, tn;
     int64_t round, step, idle, round2, step2;
 };
 static const HTile kH16Tiles[] = {
-    {"gemm", "gemm_splitk", 256, 256, 9500, 1720, 42, 9500, 1720},
+    {"gemm", "gemm_splitk", 256, 256, 10300, 1690, 50, 10300, 1690},
     {"gemm_m128", "gemm_m128_splitk", 128, 128, 3800, 487, 53, 3800, 460},
     {"gemm_m128x64", "gemm_m128x64_splitk", 128, 64, 1900, 306, 72, 1900, 360},
     {"gemm_m64", "gemm_m64_splitk", 64, 64, 1100, 210, 77, 1100, 215},
 };
 static const HTile kTcTiles[] = {
-    {"gemm_w8", "gemm_w8_splitk", 256, 256, 12500, 1900, 58, 12500, 1900},
-    {"gemm_m128", "gemm_m128_splitk", 128, 128, 5400, 857, 75, 3000, 690},
+    {"gemm_w8", "gemm_w8_splitk", 256, 256, 9800, 2250, 47, 9800, 2250},
+    {"gemm_m128", "gemm_m128_splitk", 128, 128, 5400, 720, 75, 2700, 690},
     {"gemm_m128x64", "gemm_m128x64_splitk", 128, 64, 2600, 580, 68, 2600, 640},
     {"gemm_m64", "gemm_m64_splitk", 64, 64, 1500, 370, 85, 1500, 350},
 };
@@ -632,7 +634,7 @@ static int64_t htile_cost(const HTile &ti, int64_t M, int64_t N, int64_t K, int 
     const int64_t steps = (split_chunk(K, sp) + 63) / 64;
     int64_t ns = 2600;
     if (wgs <= 256)
-        ns += ti.round + steps * ti.step * (ti.idle + (100 - ti.idle) * wgs / 256) / 100;
+        ns += (ti.round + steps * ti.step) * (ti.idle + (100 - ti.idle) * wgs / 256) / 100;
     else
         ns += (wgs + 255) / 256 * (ti.round2 + steps * ti.step2);
     if (sp > 1) ns += 2500 + (sp + 1) * M * N / 1000;
