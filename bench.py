@@ -236,7 +236,8 @@ WORKSPACE_BYTES = 2 << 30
 
 
 def shapes_leg(px, stream, reps=20, tune=True):
-    """Time the shapes that run split (phx_split_plan): each GEMM at 512^3 and
+    """Time shapes whose plan splits (phx_split_plan; a launch may run a
+    smaller tile in fewer chunks): each GEMM at 512^3 and
     1024^3, and the one-head flash .ph entry (main.rs:334-371) at 4096 x 4096.
     Inputs as in the BASELINE configs, average of `reps` launches after 3,
     under the built-in plan; with tune, also the autotuner's winner and its

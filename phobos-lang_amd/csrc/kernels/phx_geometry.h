@@ -47,7 +47,10 @@
 // are 8x cheaper, at PHX_SPLIT_TARGET_F16 workgroups with chunks of at least
 // PHX_SPLIT_MIN_STEPS_F16 steps, or PHX_SPLIT_MIN_STEPS_F16_WIDE once a
 // launch has PHX_SPLIT_WIDE_TILES tiles; at most PHX_SPLIT_MAX chunks.
-// Measured on MI355X with the partial sums in a workspace the caller bound
+// A launch that follows this rule takes a smaller tile instead, in at most as
+// many chunks, where that is estimated faster (gemm_tile_plan, s_tile_plan in
+// phx_runtime.cpp).  On the 256 x 256 tiles, between which the rule decides,
+// measured on MI355X with the partial sums in a workspace the caller bound
 // (HIP events, pinned split counts): gemm_fp16 512^3 16.6 us unsplit, 14.0
 // at 2 chunks; 768^3 20.4 / 17.1 at 3; 1536^3 33.8 / 25.8 at 3; 512^2 x
 // 2048 38.2 / 18.6 at 8; 256^2 x 4096 67.5 / 18.0 at 16; 2048^3 42.6 / 36.5
@@ -63,7 +66,8 @@
 #define PHX_SPLIT_WIDE_TILES 64
 #define PHX_SPLIT_KSTEP 32
 
-// gemm_fp32's built-in tiling (no pin): 256 x 256 x 16 when its tiles fill
+// gemm_fp32's tiling by the rule (what an unpinned launch reports, and runs
+// where its rows do not suit the smaller tiles of gemm_s_tiles.h): 256 x 256 x 16 when its tiles fill
 // all PHX_S32_FULL_TILES CUs; else 64 x 64 x 16 (launch-plan variant
 // PHX_S32_SMALL_VARIANT) when that gives at least PHX_S32_SMALL_MIN_TILES
 // tiles, or at least PHX_S32_SMALL_SHORT_TILES with K <= PHX_S32_SHORT_K;
@@ -87,7 +91,9 @@
 // run as separate workgroups (flash_attention_split) and merged by
 // flash_combine: enough chunks for PHX_FLASH_SPLIT_TARGET workgroups, of at
 // least PHX_FLASH_SPLIT_MIN_BLOCKS_F16 (f16) or _F32 (f32) blocks each, at
-// most PHX_SPLIT_MAX.  Measured on MI355X with the partial results in a
+// most PHX_SPLIT_MAX (a small-launch kernel of flash_w.h runs instead, in at
+// most as many chunks, where it is estimated faster: ftile_cost in
+// phx_runtime.cpp).  Measured on MI355X, regular kernels, with the partial results in a
 // workspace the caller bound (HIP events, pinned chunk counts; best count
 // in brackets): f16 one head 1024^2 16.2 us (3; 14.3 at 6) against 17.7 at the
 // earlier rule's 2; 8192^2 34.4 (8) against 39.4 at 16; 4 heads 4096^2 32.2
