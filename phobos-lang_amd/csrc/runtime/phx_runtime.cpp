@@ -680,7 +680,7 @@ struct SHTile {
     int64_t tm, tn, round, step[3];
 };
 static const SHTile kSTiles[] = {
-    {"gemm", "gemm_splitk", "matmul", 256, 256, 8000, {14200, 28400, 42600}},
+    {"gemm", "gemm_splitk", "matmul", 256, 256, 14000, {14200, 28400, 42600}},
     {"gemm_s64", "gemm_s64_splitk", "matmul_s64", 64, 64, 800, {930, 1800, 2680}},
     {"gemm_s64x32", "gemm_s64x32_splitk", "matmul_s64x32", 64, 32, 600, {780, 1140, 1380}},
     {"gemm_s32", "gemm_s32_splitk", "matmul_s32", 32, 32, 550, {370, 560, 780}},
@@ -717,6 +717,18 @@ static const SHTile *s_tile_plan(int64_t M, int64_t N, int64_t K, int max_sp, in
             }
         }
     return best;
+}
+
+// Whether a 64 x 64 tile of gemm_fp32 runs in K steps of 16 (gemm_t64x64k16)
+// instead of gemm_s64's 32: up to two and a half steps of 32, where starting
+// up weighs more than the step (1920 x 3008 x 64: 12.4 us against 12.8, 2112 x
+// 3520 x 72: 16.9 against 18.2, at K 96 they are equal), and for some steps
+// more where most of the last step of 32 would be padding and the CUs have
+// several tiles each (2504 x 3000 x 112: 20.7 against 21.8, 3600^2 x 144: 36.0
+// against 39.0).
+static bool s64_short_k(int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64), last = K % 32;
+    return K <= 80 || (K < 176 && last > 0 && last <= 16 && tiles > 256);
 }
 
 // Whether a launch follows the built-in plan: no environment variable forces
@@ -820,7 +832,8 @@ int launch_flash_split_ws(phx_kernel k, const Desc *t, int rank, int64_t BH, int
 // of each precision (within 8%); f16, one head of 4096^2: the wide kernel in
 // 4 chunks 14.6 us against 23.2 for the regular one in 11; 16 heads of 1000^2
 // 10.5 against 20.4; 8 heads of 512^2: 7.1 (narrow) against 13.2; 16 heads of
-// 4096^2: the regular one 84 against about 100.  f32: 4 heads of 1000 x 4133
+// 4096^2: the regular one 84 against about 100; 64 heads of 2816 x 3366: the
+// regular one 172 against 251.  f32: 16 heads of 2500 x 1500 131 against 203; 4 heads of 1000 x 4133
 // the wide kernel in 2 chunks 42.7 against 51, 16 heads of 200 x 300 11.3
 // (narrow) against 20.2.
 struct FTile {
@@ -851,7 +864,9 @@ static int64_t ftile_cost(const FTile &f, int64_t BH, int64_t Nq, int64_t Nk, in
         ns += steps * f.step;
     } else {
         const int64_t rounds = f.pair ? (n + 1) / 2 : n;
-        ns += rounds * steps * (f.pair ? f.pair : f.step) + (rounds - 1) * f.round;
+        // an odd count ends on a workgroup that has its CU to itself
+        ns += steps * (f.pair ? n / 2 * f.pair + n % 2 * f.step : n * f.step) +
+              (rounds - 1) * f.round;
     }
     if (sp > 1) ns += 2300 + sp * BH * Nq * 264 / 2300;
     return ns;
@@ -975,6 +990,9 @@ int launch_raw(hipFunction_t f, const uint32_t grid[3], const uint32_t block[3],
                     const SHTile *ti = s_tile_plan(d[0], d[1], d[2], sp, &msp);
                     entry = ti->entry, split_entry = ti->split_entry, tm = ti->tm, tn = ti->tn;
                     cap = kSTileGrid;
+                    if (tm == 64 && tn == 64 && msp == 1 && s64_short_k(d[0], d[1], d[2]))
+                        return launch_tiled(kSpecs[k].file, kS32[PHX_S32_SMALL_VARIANT].entry, tm,
+                                            tn, PHX_S_THREADS, 0, d[0], d[1], s, args);
                 } else {
                     const HTile *ti = gemm_tile_plan((phx_kernel)k, d[0], d[1], d[2], sp, &msp);
                     entry = ti->entry, split_entry = ti->split_entry, tm = ti->tm, tn = ti->tn;

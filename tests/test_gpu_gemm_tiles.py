@@ -115,7 +115,7 @@ def test_each_tile_meets_the_oracle(px_gpu, stream, kern_name, M, N, K, pad):
 @pytest.mark.parametrize("kern_name", list(KERNELS))
 @pytest.mark.parametrize("M,N,K", [(64, 64, 4096), (65, 72, 2056), (200, 520, 3000),
                                    (1000, 1000, 1000), (1208, 1208, 64), (300, 4096, 512),
-                                   (2100, 2056, 40)])
+                                   (2100, 2056, 40), (1100, 1064, 104)])
 def test_rule_launches_meet_the_oracle(px_gpu, stream, kern_name, M, N, K):
     # through the built-in plan: the tile it picks, split over K into the
     # bound workspace where that is cheaper, and on a stream without one
