@@ -19,6 +19,12 @@
 #pragma once
 
 #define FW_PITCH 68  // floats per query in the merge
+// A key group's running max before its first block, and the least it takes
+// there: finite, so that a block of -inf scores only weighs 0 and not
+// exp2(-inf + inf).  M_INIT will not do: a group may start on a block whose
+// scores all lie below it (keys a caller pads with a large negative value), and
+// 2^(M_INIT - max) then overflows.
+#define FW_M0 (-3.402823466e38f)
 
 // Merges the key groups' sums of a workgroup of QW x KG waves (wave = grp * QW
 // + query tile): O = sum_g 2^(m_g - M) acc_g / sum_g 2^(m_g - M) l_g.  The first

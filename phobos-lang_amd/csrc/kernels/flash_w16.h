@@ -64,12 +64,16 @@ __device__ __forceinline__ void w16_step(Flash16 &fs, KFrag &kf, char *Vs, const
     }
     if (slow) {
         const float mx = row_max(sc) * c2;  // log2 units
-        const float m2n = FIRST || mx > fs.m2 + RESCALE_SLACK ? mx : fs.m2;
+        const float m2n = FIRST                            ? fmaxf(mx, FW_M0)
+                          : mx > fs.m2 + RESCALE_SLACK ? mx
+                                                       : fs.m2;
         ps = softmax_p(pf, sc, c2, m2n);
-        const float corr = __builtin_amdgcn_exp2f(fs.m2 - m2n);  // 1 where not raised
-        fs.l = fs.l * corr;
-        fs.acc[0] = fs.acc[0] * corr;
-        fs.acc[1] = fs.acc[1] * corr;
+        if (!FIRST) {
+            const float corr = __builtin_amdgcn_exp2f(fs.m2 - m2n);  // 1 where not raised
+            fs.l = fs.l * corr;
+            fs.acc[0] = fs.acc[0] * corr;
+            fs.acc[1] = fs.acc[1] * corr;
+        }
         fs.m2 = m2n;
     }
     fs.l += ps;
@@ -117,7 +121,7 @@ __device__ __forceinline__ void w16_block(const T *Q, const T *Kp, const T *Vp, 
     }
     fs.acc[0] = (phx_f16v){0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     fs.acc[1] = fs.acc[0];
-    fs.m2 = M_INIT * LOG2E;  // replaced by the first block's row max
+    fs.m2 = FW_M0;  // replaced by the first block's row max, if the group has one
     fs.l = 0.0f;
 #define W16S(F, S, KF, I) w16_step<KG, F>(fs, KF, S, Kp, Vp, ldk, ldv, Nk, I, c2, vk, vv, lane)
     uint32_t i = wave;
@@ -181,12 +185,16 @@ __device__ __forceinline__ void w2_step(Flash16 &fs, const char *cur, char *fill
     }
     if (slow) {
         const float mx = row_max(sc) * c2;  // log2 units
-        const float m2n = FIRST || mx > fs.m2 + RESCALE_SLACK ? mx : fs.m2;
+        const float m2n = FIRST                            ? fmaxf(mx, FW_M0)
+                          : mx > fs.m2 + RESCALE_SLACK ? mx
+                                                       : fs.m2;
         ps = softmax_p(pf, sc, c2, m2n);
-        const float corr = __builtin_amdgcn_exp2f(fs.m2 - m2n);  // 1 where not raised
-        fs.l = fs.l * corr;
-        fs.acc[0] = fs.acc[0] * corr;
-        fs.acc[1] = fs.acc[1] * corr;
+        if (!FIRST) {
+            const float corr = __builtin_amdgcn_exp2f(fs.m2 - m2n);  // 1 where not raised
+            fs.l = fs.l * corr;
+            fs.acc[0] = fs.acc[0] * corr;
+            fs.acc[1] = fs.acc[1] * corr;
+        }
         fs.m2 = m2n;
     }
     fs.l += ps;
@@ -238,7 +246,7 @@ __device__ __forceinline__ void w2_block(const T *Q, const T *Kp, const T *Vp, T
     }
     fs.acc[0] = (phx_f16v){0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     fs.acc[1] = fs.acc[0];
-    fs.m2 = M_INIT * LOG2E;  // replaced by the first block's row max
+    fs.m2 = FW_M0;  // replaced by the first block's row max, if the group has one
     fs.l = 0.0f;
     // the groups take blocks grp, grp + KG, ... in step, so every wave meets
     // every barrier; a group past its last block skips the work

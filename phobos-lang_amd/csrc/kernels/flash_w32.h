@@ -77,7 +77,7 @@ __device__ __forceinline__ void w32_step(W32 &w, const T *Kp, const T *Vp, int64
     for (int r = 1; r < 16; ++r) mx = fmaxf(mx, p[r]);
     mx = xor32_max(mx) * c2;
     const bool raise = first || mx > w.m2 + RESCALE_SLACK;
-    const float m2n = raise ? mx : w.m2;
+    const float m2n = raise ? fmaxf(mx, FW_M0) : w.m2;
     float part[4];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
@@ -127,7 +127,7 @@ __device__ __forceinline__ void w32_block(const T *Q, const T *Kp, const T *Vp, 
     w32_load_v(w, Vp, ldv, Nk, wave, vv);
     w.acc[0] = (phx_f16v){0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     w.acc[1] = w.acc[0];
-    w.m2 = M_INIT * LOG2E;
+    w.m2 = FW_M0;
     w.l = 0.0f;
     // this wave's steps: wave, wave + KG, ...
     for (uint32_t i = wave; i < n32; i += KG)
