@@ -54,7 +54,8 @@ __device__ __forceinline__ void fw_merge(const phx_f16v (&acc)[2], float m2, flo
     constexpr uint32_t TPQ = 64 * NW / NQ, NV = 64 / TPQ / 4;  // threads per query, float4s each
     const uint32_t qt = tid / TPQ, d0 = (tid % TPQ) * (4 * NV), q = q0 + qt;
     const uint32_t ql = qt % 32, w0 = qt / 32;  // the query's place in waves w0, w0 + QW, ...
-    float mw[KG], M = M_INIT * LOG2E, l = 0.0f;
+    // from the groups' own maxima: a group without a block carries FW_M0 and l = 0
+    float mw[KG], M = FW_M0, l = 0.0f;
 #pragma unroll
     for (int x = 0; x < KG; ++x) {
         mw[x] = ml[((w0 + x * QW) * 32 + ql) * 2];

@@ -115,3 +115,39 @@ def test_planned_launch_with_padded_keys(px_gpu, stream, bits):
     got = (oracle.f16_to_f32(do.download(np.uint16, Nq * D)).reshape(Nq, D) if bits == 16
            else do.download(np.float32, (Nq, D)))
     assert _rel(got, _softmax(q[None], k[None], v[None], 0.125)[0]) < TOL[bits]
+
+
+@pytest.mark.parametrize("bits,entry", _all_entries())
+@pytest.mark.parametrize("Nk", [1, 40, 100, 320, 520])
+def test_every_key_far_below_the_initial_max(px_gpu, stream, bits, entry, Nk):
+    # every score is -102400 (f16) or -6.4e8 (f32), in f16 one key's 3.75 more
+    # (the scores are exact; a max of this size in log2 units is rounded by up
+    # to 2^-7, which weighs its group 0.5% wrong), in groups with blocks and
+    # without (Nk under KG steps)
+    px, (qv, kv), scale = px_gpu, ((40.0, -40.0) if bits == 16 else (1e3, -1e4)), 1.0
+    q, k, v = _inputs(bits, 2, 33, Nk, 151)
+    q[:], k[:] = qv, kv
+    if bits == 16:
+        k[:, Nk // 2, 0] += 3.0 / 32.0
+    e = _Entry(px, stream, bits, entry, q, k, v, scale)
+    want = _softmax(q, k, v, scale)
+    for sp in (1, 2, 3):
+        assert _rel(e.run(sp), want) < TOL[bits], sp
+    e.close()
+
+
+@pytest.mark.parametrize("bits", [16, 32])
+def test_planned_launch_far_below_the_initial_max(px_gpu, stream, bits):
+    px, (qv, kv) = px_gpu, ((40.0, -40.0) if bits == 16 else (1e3, -1e4))
+    Nq, Nk = 32, 200
+    v = _inputs(bits, 1, 1, Nk, 161)[2][0]
+    q, k = np.full((Nq, D), qv, np.float32), np.full((Nk, D), kv, np.float32)
+    up = oracle.f16_bits if bits == 16 else np.ascontiguousarray
+    dq, dk, dv = (px.DeviceBuffer.from_array(up(t)) for t in (q, k, v))
+    do = px.DeviceBuffer(Nq * D * bits // 8)
+    px.launch_flash(stream, px.FLASH_FP16 if bits == 16 else px.FLASH_FP32, dq, dk, dv, do, Nq, Nk,
+                    D, 1.0)
+    stream.synchronize()
+    got = (oracle.f16_to_f32(do.download(np.uint16, Nq * D)).reshape(Nq, D) if bits == 16
+           else do.download(np.float32, (Nq, D)))
+    assert _rel(got, np.broadcast_to(v.astype(np.float64).mean(axis=0), got.shape)) < TOL[bits]
