@@ -861,11 +861,12 @@ extern "C" __global__ __launch_bounds__(256) void flash_combine(const float *W, 
             acc = acc * c;
             mx = m4;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const float w = s0 + u < nsplit ? __builtin_amdgcn_exp2f(v[u].x - mx) : 0.0f;
-                l = l + w * v[u].y;
-                acc = acc + w * a[u];
-            }
+            for (int u = 0; u < 4; ++u)
+                if (s0 + u < nsplit) {  // uniform; no 0 * a: a may be infinite
+                    const float w = __builtin_amdgcn_exp2f(v[u].x - mx);
+                    l = l + w * v[u].y;
+                    acc = acc + w * a[u];
+                }
         }
         const int64_t h = hqi / Nq, q = hqi % Nq;
         T *dst = O + h * ho + q * ldo + 4 * d4;

@@ -151,3 +151,28 @@ def test_planned_launch_far_below_the_initial_max(px_gpu, stream, bits):
     got = (oracle.f16_to_f32(do.download(np.uint16, Nq * D)).reshape(Nq, D) if bits == 16
            else do.download(np.float32, (Nq, D)))
     assert _rel(got, np.broadcast_to(v.astype(np.float64).mean(axis=0), got.shape)) < TOL[bits]
+
+
+@pytest.mark.parametrize("bits", [16, 32])
+@pytest.mark.parametrize("splits", [1, 2, 3, 4, 5, 6, 7])
+def test_an_infinite_value_stays_infinite(px_gpu, stream, monkeypatch, bits, splits):
+    # V holds one infinity per sign: every output of its column is that
+    # infinity, whatever the number of chunks flash_combine merges (it reads
+    # them in batches of four)
+    px = px_gpu
+    monkeypatch.setenv("PHX_FLASH_SPLIT", str(splits))
+    Nq, Nk = 40, 448
+    q, k, v = (t[0] for t in _inputs(bits, 1, Nq, Nk, 171))
+    v[3, 5], v[440, 9] = np.inf, -np.inf
+    up = oracle.f16_bits if bits == 16 else np.ascontiguousarray
+    dq, dk, dv = (px.DeviceBuffer.from_array(up(t)) for t in (q, k, v))
+    do = px.DeviceBuffer(Nq * D * bits // 8)
+    px.launch_flash(stream, px.FLASH_FP16 if bits == 16 else px.FLASH_FP32, dq, dk, dv, do, Nq, Nk,
+                    D, 0.125)
+    stream.synchronize()
+    got = (oracle.f16_to_f32(do.download(np.uint16, Nq * D)).reshape(Nq, D) if bits == 16
+           else do.download(np.float32, (Nq, D)))
+    assert (got[:, 5] == np.inf).all() and (got[:, 9] == -np.inf).all()
+    rest = [d for d in range(D) if d not in (5, 9)]
+    want = _softmax(q[None], k[None], v[None][:, :, rest], 0.125)[0]
+    assert _rel(got[:, rest], want) < TOL[bits]
