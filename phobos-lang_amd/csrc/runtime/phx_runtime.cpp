@@ -611,21 +611,36 @@ static int gemm_split_fit(int sp, int64_t M, int64_t N, int64_t K, size_t cap) {
 struct HTile {
     const char *entry, *split_entry;
     int64_t tm, tn;
+    int sets;  // accumulator sets
     int64_t round, step, idle, round2, step2;
 };
 static const HTile kH16Tiles[] = {
-    {"gemm", "gemm_splitk", 256, 256, 10300, 1690, 50, 10300, 1690},
-    {"gemm_m128", "gemm_m128_splitk", 128, 128, 3800, 487, 53, 3800, 460},
-    {"gemm_m128x64", "gemm_m128x64_splitk", 128, 64, 1900, 306, 72, 1900, 360},
-    {"gemm_m64", "gemm_m64_splitk", 64, 64, 1100, 210, 77, 1100, 215},
+    {"gemm", "gemm_splitk", 256, 256, 1, 10300, 1690, 50, 10300, 1690},
+    {"gemm_m128", "gemm_m128_splitk", 128, 128, 1, 3800, 487, 53, 3800, 460},
+    {"gemm_m128x64", "gemm_m128x64_splitk", 128, 64, 2, 1900, 306, 72, 1900, 360},
+    {"gemm_m64", "gemm_m64_splitk", 64, 64, 4, 1100, 210, 77, 1100, 215},
 };
 static const HTile kTcTiles[] = {
-    {"gemm_w8", "gemm_w8_splitk", 256, 256, 9800, 2250, 47, 9800, 2250},
-    {"gemm_m128", "gemm_m128_splitk", 128, 128, 5400, 720, 75, 2700, 690},
-    {"gemm_m128x64", "gemm_m128x64_splitk", 128, 64, 2600, 580, 68, 2600, 640},
-    {"gemm_m64", "gemm_m64_splitk", 64, 64, 1500, 370, 85, 1500, 350},
+    {"gemm_w8", "gemm_w8_splitk", 256, 256, 1, 9800, 2250, 47, 9800, 2250},
+    {"gemm_m128", "gemm_m128_splitk", 128, 128, 2, 5400, 720, 75, 2700, 690},
+    {"gemm_m128x64", "gemm_m128x64_splitk", 128, 64, 4, 2600, 580, 68, 2600, 640},
+    {"gemm_m64", "gemm_m64_splitk", 64, 64, 4, 1500, 370, 85, 1500, 350},
 };
 constexpr int kHTiles = 4;
+
+// What the f32 sum of an output's K products gathers in rounding errors, as a
+// variance in half matrix instructions: 2 per instruction of a chain
+// (`products` summed by each), `sets` chains per wave added in pairs,
+// `shares` of K in as many waves and `sp` chunks added in turn.  Against f64
+// (tc 1536^2 x 4096: 2.06e-7 as 3 chunks of the 256 x 256 tile, 2.89e-7 as
+// two chains of 2048; 1304 x 728 x 1864: 1.21e-7 in 7, 1.45e-7 as four of 466;
+// 1760 x 448 x 2840: 1.30e-7 in 9, 1.75e-7) its square root gives the ratios
+// within 3%.
+static int64_t sum_noise(int64_t K, int sp, int sets, int shares, int products) {
+    const int64_t n = (int64_t)sets * shares * products;
+    return 2 * ((split_chunk(K, sp) + n - 1) / n) + (sets > 2 ? 4 : sets > 1 ? 2 : 0) +
+           (shares > 1 ? shares : 0) + (sp > 1 ? sp : 0);
+}
 
 // Estimated nanoseconds of a launch on tile ti in sp K chunks.  A split adds
 // its reduce kernel: about 2.5 us and the f32 planes at 4 TB/s.
@@ -643,11 +658,15 @@ static int64_t htile_cost(const HTile &ti, int64_t M, int64_t N, int64_t K, int 
 
 // The tile and K split of a gemm_fp16 or gemm_fp16tc_fp32acc launch that
 // follows the built-in plan: the cheapest of every tile in every split up to
-// max_sp chunks (the built-in plan's, cut to the bound workspace).
+// max_sp chunks (the built-in plan's, cut to the bound workspace), for
+// gemm_fp16tc_fp32acc of those whose sums are no less exact than the 256 x
+// 256 tile's in max_sp chunks (gemm_fp16 rounds them to f16, where no plan's
+// error differs: 2.07e-4 for each).
 static const HTile *gemm_tile_plan(phx_kernel k, int64_t M, int64_t N, int64_t K, int max_sp,
                                    int *splits) {
     const HTile *tiles = k == PHX_GEMM_FP16 ? kH16Tiles : kTcTiles;
     const int64_t units = (K + PHX_SPLIT_KSTEP - 1) / PHX_SPLIT_KSTEP;
+    const int64_t noise = sum_noise(K, max_sp, 1, 1, 16);
     const HTile *best = nullptr;
     int64_t least = 0;
     for (int i = 0; i < kHTiles; ++i)
@@ -655,6 +674,7 @@ static const HTile *gemm_tile_plan(phx_kernel k, int64_t M, int64_t N, int64_t K
             const int sp = want == 1 ? 1 : round_split(units, want);
             if (sp == last) continue;
             last = sp;
+            if (k != PHX_GEMM_FP16 && sum_noise(K, sp, tiles[i].sets, 1, 16) > noise) continue;
             const int64_t ns = htile_cost(tiles[i], M, N, K, sp);
             if (!best || ns < least) {
                 best = &tiles[i];
@@ -677,13 +697,15 @@ static const HTile *gemm_tile_plan(phx_kernel k, int64_t M, int64_t N, int64_t K
 // (926; 945 for 64 x 64).
 struct SHTile {
     const char *entry, *split_entry, *leaf;
-    int64_t tm, tn, round, step[3];
+    int64_t tm, tn;
+    int sets, shares;  // accumulators of a wave, waves sharing K (sum_noise)
+    int64_t round, step[3];
 };
 static const SHTile kSTiles[] = {
-    {"gemm", "gemm_splitk", "matmul", 256, 256, 14000, {14200, 28400, 42600}},
-    {"gemm_s64", "gemm_s64_splitk", "matmul_s64", 64, 64, 800, {930, 1800, 2680}},
-    {"gemm_s64x32", "gemm_s64x32_splitk", "matmul_s64x32", 64, 32, 600, {780, 1140, 1380}},
-    {"gemm_s32", "gemm_s32_splitk", "matmul_s32", 32, 32, 550, {370, 560, 780}},
+    {"gemm", "gemm_splitk", "matmul", 256, 256, 1, 1, 14000, {14200, 28400, 42600}},
+    {"gemm_s64", "gemm_s64_splitk", "matmul_s64", 64, 64, 2, 1, 800, {930, 1800, 2680}},
+    {"gemm_s64x32", "gemm_s64x32_splitk", "matmul_s64x32", 64, 32, 2, 2, 600, {780, 1140, 1380}},
+    {"gemm_s32", "gemm_s32_splitk", "matmul_s32", 32, 32, 2, 4, 550, {370, 560, 780}},
 };
 // Workgroups a small f32 tile's launch starts at most, walking the tiles with
 // that stride: the three per CU that are resident at once (at 2048^3 the 64 x
@@ -700,8 +722,11 @@ static int64_t stile_cost(const SHTile &ti, int64_t M, int64_t N, int64_t K, int
     return ns;
 }
 
+// The cheapest tile and split, as gemm_tile_plan; f32 sums, so never a less
+// exact one than the 256 x 256 tile's in max_sp chunks.
 static const SHTile *s_tile_plan(int64_t M, int64_t N, int64_t K, int max_sp, int *splits) {
     const int64_t units = (K + PHX_SPLIT_KSTEP - 1) / PHX_SPLIT_KSTEP;
+    const int64_t noise = sum_noise(K, max_sp, 1, 1, 2);
     const SHTile *best = nullptr;
     int64_t least = 0;
     for (const SHTile &ti : kSTiles)
@@ -709,6 +734,7 @@ static const SHTile *s_tile_plan(int64_t M, int64_t N, int64_t K, int max_sp, in
             const int sp = want == 1 ? 1 : round_split(units, want);
             if (sp == last) continue;
             last = sp;
+            if (sum_noise(K, sp, ti.sets, ti.shares, 2) > noise) continue;
             const int64_t ns = stile_cost(ti, M, N, K, sp);
             if (!best || ns < least) {
                 best = &ti;
@@ -725,7 +751,8 @@ static const SHTile *s_tile_plan(int64_t M, int64_t N, int64_t K, int max_sp, in
 // 3520 x 72: 16.9 against 18.2, at K 96 they are equal), and for some steps
 // more where most of the last step of 32 would be padding and the CUs have
 // several tiles each (2504 x 3000 x 112: 20.7 against 21.8, 3600^2 x 144: 36.0
-// against 39.0).
+// against 39.0).  It sums K in one chain, so it stands in only where the
+// built-in plan does not split.
 static bool s64_short_k(int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64), last = K % 32;
     return K <= 80 || (K < 176 && last > 0 && last <= 16 && tiles > 256);
@@ -990,7 +1017,7 @@ int launch_raw(hipFunction_t f, const uint32_t grid[3], const uint32_t block[3],
                     const SHTile *ti = s_tile_plan(d[0], d[1], d[2], sp, &msp);
                     entry = ti->entry, split_entry = ti->split_entry, tm = ti->tm, tn = ti->tn;
                     cap = kSTileGrid;
-                    if (tm == 64 && tn == 64 && msp == 1 && s64_short_k(d[0], d[1], d[2]))
+                    if (tm == 64 && tn == 64 && sp == 1 && s64_short_k(d[0], d[1], d[2]))
                         return launch_tiled(kSpecs[k].file, kS32[PHX_S32_SMALL_VARIANT].entry, tm,
                                             tn, PHX_S_THREADS, 0, d[0], d[1], s, args);
                 } else {

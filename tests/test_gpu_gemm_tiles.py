@@ -145,3 +145,33 @@ def test_rows_that_overlap_run_the_256_tile(px_gpu, stream):
                                  stream.handle, arr))
     stream.synchronize()
     _check(case, case.dev[2].download(case.dt, case.host[2].shape), 1.0, 0.0)
+
+
+# extents whose built-in split has shorter chains than a small tile's
+# accumulator sets would have
+@pytest.mark.parametrize("kern_name,M,N,K", [
+    ("GEMM_FP16TC_FP32ACC", 1536, 1536, 4096), ("GEMM_FP16TC_FP32ACC", 1304, 728, 1864),
+    ("GEMM_FP16TC_FP32ACC", 1760, 448, 2840), ("GEMM_FP16TC_FP32ACC", 284, 2528, 3432),
+    ("GEMM_FP16TC_FP32ACC", 1280, 1280, 1280), ("GEMM_FP16TC_FP32ACC", 1000, 1000, 1000),
+    ("GEMM_FP32", 400, 96, 376), ("GEMM_FP32", 113, 104, 400), ("GEMM_FP32", 564, 64, 392),
+    ("GEMM_FP32", 96, 80, 344)])
+def test_small_tiles_sum_no_less_exactly_than_the_split(px_gpu, stream, monkeypatch, kern_name, M,
+                                                        N, K):
+    # root mean square error against f64 of the tile the built-in plan picks
+    # and of the split it names on the 256 x 256 tile: within 5% (the root mean
+    # square of 7680 errors scatters by 1%, and sum_noise fits within 3%)
+    px = px_gpu
+    kern = getattr(px, kern_name)
+    case = _Case(px, kern, M, N, K, 0)
+    ref = case.A.astype(np.float64) @ case.B.astype(np.float64)
+    fn = px.builtin_function(kern)
+
+    def rms():
+        got = case.values(case.launch(stream, fn, 1, 256, 1.0, 0.0)).reshape(ref.shape)
+        return np.sqrt(np.mean((got - ref) ** 2))
+
+    splits = px.split_plan(kern, [M, N, K])[0]
+    assert splits > 1
+    picked = rms()
+    monkeypatch.setenv("PHX_GEMM_SPLIT", str(splits))
+    assert picked <= 1.05 * rms()
