@@ -14,9 +14,10 @@ the 256 MB MALL, which the next plan would then pay for).  The space here
 is the launch plan (phx_plan): the number of K chunks of a GEMM or key
 chunks of a flash launch, gemm_fp32's tile dims (TILE_M x TILE_N x TILE_K
 over the reference's ranges), and for gemm_fp16tc_fp32acc which of its
-two kernel families (eight-wave or one-wave) runs.  The winner is pinned
-with phx_plan_pin, so every later launch of that kernel at that shape uses
-it.
+two kernel families (eight-wave or one-wave) runs.  The built-in plan is
+always searched (with_rule): a launch pinned to it runs as one without a
+pin, smaller tiles included.  The winner is pinned with phx_plan_pin, so
+every later launch of that kernel at that shape uses it.
 
 A candidate is verified on its first launch against the unsplit plan's
 output (a split changes only the order of the f32 sums): relative to the
@@ -30,7 +31,7 @@ import numpy as np
 from . import (FLASH_FP16, FLASH_FP16_BH, FLASH_FP32_BH, GEMM_FP16, GEMM_FP16TC_FP32ACC,
                GEMM_FP32, GEMM_FP32_TILINGS,
                DeviceBuffer, Event, PhxError, bind_workspace, get_workspace, launch_flash,
-               launch_flash_bh, launch_gemm, normal_f32, plan_pin, to_f16_bits)
+               launch_flash_bh, launch_gemm, normal_f32, plan_get, plan_pin, to_f16_bits)
 
 SPLITS = (1, 2, 3, 4, 6, 8, 12, 16)  # the split counts a search tries
 MAX_WORKSPACE = 4 << 30               # skip splits whose partial sums need more
@@ -107,6 +108,17 @@ def flash_space(BH, Nq, Nk):
         if (e, 0) not in space and (e == 1 or e * BH * Nq * 66 * 4 <= MAX_WORKSPACE):
             space.append((e, 0))
     return space
+
+
+def with_rule(kernel, dims, space):
+    """space, and the built-in plan where its chunk count is not among those
+    tried (gemm_fp16 at 1280^3: 5).  The plan equal to the built-in one is the
+    only one under which a launch may take a smaller tile or a small-launch
+    flash kernel, so a search without it could pin a plan slower than none.
+    Takes off any pin of these dims."""
+    plan_pin(kernel, dims, None)
+    rule = tuple(plan_get(kernel, dims))
+    return space if rule in space else space + [rule]
 
 
 class Autotuner:
@@ -200,8 +212,9 @@ def _close(got, want, tol):
 
 
 def tune_gemm(stream, kernel, M, N, K, alpha=1.0, beta=0.0, seed=1, **kw):
-    """Searches gemm_space for kernel at M x N x K (row-major, alpha, beta as
-    the caller launches it) on seeded inputs and pins the winner."""
+    """Searches gemm_space and the built-in plan for kernel at M x N x K
+    (row-major, alpha, beta as the caller launches it) on seeded inputs and
+    pins the winner."""
     f16 = kernel == GEMM_FP16
     esz = 2 if f16 else 4
     conv = (lambda x: to_f16_bits(x)) if f16 else (lambda x: x.astype(np.float32))
@@ -222,6 +235,7 @@ def tune_gemm(stream, kernel, M, N, K, alpha=1.0, beta=0.0, seed=1, **kw):
         r = C.download(out_dtype, M * N)
         return r.view(np.float16).astype(np.float32) if f16 else r
 
+    space = with_rule(kernel, dims, gemm_space(kernel, M, N, K))
     plan_pin(kernel, dims, 1, 0)
     C.upload(c0)
     run_once()
@@ -236,16 +250,16 @@ def tune_gemm(stream, kernel, M, N, K, alpha=1.0, beta=0.0, seed=1, **kw):
         _close(result(), want, tol)
 
     reset = None if beta == 0.0 else (lambda: C.upload(c0))
-    space = gemm_space(kernel, M, N, K)
     ensure_workspace(stream, max(sp for sp, _ in space) * M * N * 4)
     tuner = Autotuner(stream, kernel, dims, run_once, verify, reset=reset, **kw)
     return tuner.run(space)
 
 
 def tune_flash(stream, kernel, BH, Nq, Nk, D=64, scale=0.125, seed=1, **kw):
-    """Searches flash_space for kernel (one-head or batched, f16 or f32) at
-    BH heads x Nq queries x Nk keys on seeded N(0,1) inputs; pins the winner
-    (shared by the one-head and batched kernels of the precision)."""
+    """Searches flash_space and the built-in plan for kernel (one-head or
+    batched, f16 or f32) at BH heads x Nq queries x Nk keys on seeded N(0,1)
+    inputs; pins the winner (shared by the one-head and batched kernels of the
+    precision)."""
     f16 = kernel in (FLASH_FP16, FLASH_FP16_BH)
     bh = kernel in (FLASH_FP16_BH, FLASH_FP32_BH)
     if not bh and BH != 1:
@@ -267,6 +281,7 @@ def tune_flash(stream, kernel, BH, Nq, Nk, D=64, scale=0.125, seed=1, **kw):
         r = O.download(np.uint16 if f16 else np.float32, BH * Nq * D)
         return r.view(np.float16).astype(np.float32) if f16 else r
 
+    space = with_rule(kernel, dims, flash_space(BH, Nq, Nk))
     plan_pin(kernel, dims, 1, 0)
     launch()
     stream.synchronize()
@@ -276,7 +291,6 @@ def tune_flash(stream, kernel, BH, Nq, Nk, D=64, scale=0.125, seed=1, **kw):
     def verify():
         _close(result(), want, tol)
 
-    space = flash_space(BH, Nq, Nk)
     ensure_workspace(stream, max(sp for sp, _ in space) * BH * Nq * (D + 2) * 4)
     tuner = Autotuner(stream, kernel, dims, launch, verify, **kw)
     return tuner.run(space)

@@ -64,3 +64,29 @@ def test_flash_space():
     assert autotune.flash_space(1, 4096, 4096) == [(1, 0), (2, 0), (3, 0), (4, 0), (6, 0),
                                                    (8, 0), (11, 0), (16, 0)]
     assert autotune.flash_space(1, 64, 100) == [(1, 0), (2, 0)]  # two key blocks
+
+
+def test_the_built_in_plan_is_always_searched():
+    # whatever chunk count the rule names (5, 7, 9, ... are not in SPLITS), and
+    # with a pin of the shape in place
+    import phobos_amd as px
+    sizes = (64, 200, 304, 512, 640, 768, 1000, 1280, 1536, 1800, 2048, 4096)
+    counts = set()
+    for M, N, K in itertools.product(sizes, sizes, sizes):
+        for kern in (GEMM_FP32, GEMM_FP16TC_FP32ACC, GEMM_FP16):
+            rule = px.plan_get(kern, [M, N, K])
+            space = autotune.gemm_space(kern, M, N, K)
+            got = autotune.with_rule(kern, [M, N, K], space)
+            assert rule in got and got[:len(space)] == space and len(got) == len(set(got))
+            counts.add(rule[0])
+    assert counts - set(autotune.SPLITS)
+    for BH, Nq, Nk in itertools.product((1, 3, 16), sizes, sizes):
+        for kern in (px.FLASH_FP16_BH, px.FLASH_FP32_BH):
+            dims = [BH, Nq, Nk, 64]
+            assert px.plan_get(kern, dims) in autotune.with_rule(kern, dims,
+                                                                 autotune.flash_space(BH, Nq, Nk))
+    dims = [1280, 1280, 1280]
+    rule = px.plan_get(GEMM_FP16, dims)
+    px.plan_pin(GEMM_FP16, dims, 3)
+    assert rule in autotune.with_rule(GEMM_FP16, dims, [(1, 0)])
+    px.plan_unpin_all()

@@ -165,3 +165,19 @@ def test_tune_flash_pins_a_correct_winner(px_gpu, stream, bits):
     rows = np.unique(np.linspace(0, Nq - 1, 32).astype(np.int64))
     want = oracle.flash_rows(rows, q, k, v, 0.125)
     assert (np.abs(got[rows] - want) / np.maximum(np.abs(want), 0.1)).max() < (2e-2 if bits == 16 else 1e-4)
+
+
+def test_tuned_launch_is_not_slower_than_an_unpinned_one(px_gpu, stream):
+    # gemm_fp16 1280^3: the built-in plan names 5 chunks, which SPLITS does not
+    # have, and runs a smaller tile unsplit; every other plan of the search
+    # runs the 256 x 256 tile at about twice its time
+    from phobos_amd import autotune
+    px = px_gpu
+    kern, dims = px.GEMM_FP16, [1280, 1280, 1280]
+    rule = px.plan_get(kern, dims)
+    assert rule not in autotune.gemm_space(kern, *dims)
+    r = autotune.tune_gemm(stream, kern, *dims, short_probes=2, long_probes=4, finalists=2)
+    us = {tuple(s["plan"]): s["us"] for s in r["stage1"]}
+    assert us[rule] == min(us.values()) and tuple(r["winner"]) == rule
+    run, want = _gemm_case(px, stream, kern, *dims)
+    _gemm_ok(px, kern, run(), want)
