@@ -924,7 +924,9 @@ int launch_flash_small(phx_kernel k, const Desc *t, int rank, int64_t BH, int64_
     const FTile *best = nullptr;
     int64_t least = ftile_cost(tiles[0], BH, Nq, Nk, max_sp);
     int32_t sp = 1;
-    for (int i = 1; i < 3; ++i)
+    for (int i = 1; i < 3; ++i) {
+        // one workgroup per item, of less than 2^32 threads in all
+        if ((Nq + tiles[i].q - 1) / tiles[i].q * BH > UINT32_MAX / tiles[i].threads) continue;
         for (int want = 1, last = 0; want <= max_sp; ++want) {
             const int c = want == 1 ? 1 : round_split(nkb, want);
             if (c == last) continue;
@@ -936,6 +938,7 @@ int launch_flash_small(phx_kernel k, const Desc *t, int rank, int64_t BH, int64_
                 sp = c;
             }
         }
+    }
     if (!best) return PHX_OK;
     hipFunction_t f, fc = nullptr;
     if (int rc = aux_function(kSpecs[k].file, best->entry, &f)) return rc;
@@ -963,14 +966,17 @@ static int flash_split_fit(int sp, int64_t BH, int64_t Nq, int64_t Nk, size_t ca
 }
 
 // One workgroup of `threads` per tm x tn output tile, at most cap of them
-// (0: any number), of a GEMM entry that takes the .ph kernel's own argument
-// list and walks the tiles with the grid's stride.
+// (0: as many as a launch takes, less than 2^32 threads), of a GEMM entry that
+// takes the .ph kernel's own argument list and walks the tiles with the grid's
+// stride.
 static int launch_tiled(const char *file, const char *entry, int64_t tm, int64_t tn,
-                        uint32_t threads, uint32_t cap, int64_t M, int64_t N, hipStream_t s, void **args) {
+                        uint32_t threads, uint32_t cap, int64_t M, int64_t N, hipStream_t s,
+                        void **args) {
     hipFunction_t f;
     if (int rc = aux_function(file, entry, &f)) return rc;
     const int64_t tiles = ((M + tm - 1) / tm) * ((N + tn - 1) / tn);
-    const uint32_t grid = (uint32_t)(cap && tiles > cap ? cap : tiles);
+    if (!cap) cap = UINT32_MAX / threads;
+    const uint32_t grid = (uint32_t)(tiles > cap ? cap : tiles);
     hipError_t e = hipModuleLaunchKernel(f, grid, 1, 1, threads, 1, 1, 0, s, args, nullptr);
     return e == hipSuccess ? PHX_OK : hip_error(e, "hipModuleLaunchKernel(gemm tile)");
 }

@@ -175,3 +175,30 @@ def test_small_tiles_sum_no_less_exactly_than_the_split(px_gpu, stream, monkeypa
     picked = rms()
     monkeypatch.setenv("PHX_GEMM_SPLIT", str(splits))
     assert picked <= 1.05 * rms()
+
+
+def test_more_tiles_than_a_launch_takes_workgroups(px_gpu, stream):
+    # 2^31 - 1 rows of gemm_fp16 in 128 x 64 tiles would be 2^24 workgroups of
+    # 256 threads, one more than a launch takes; A of equal elements, so every
+    # row of C is the same, over a C of NaN (32 GiB each, checked at both ends
+    # and in between)
+    px = px_gpu
+    M, N, K = 2 ** 31 - 1, 8, 8
+    dA, dC = px.DeviceBuffer(M * K * 2), px.DeviceBuffer(M * N * 2)
+    px.check(px.lib().phx_memset_async(dA.ptr, 0x38, M * K * 2, None))
+    px.check(px.lib().phx_memset_async(dC.ptr, 0xFF, M * N * 2, None))
+    px.synchronize()
+    B = (np.arange(K * N, dtype=np.float32) / 8).reshape(K, N)
+    dB = px.DeviceBuffer.from_array(oracle.f16_bits(B))
+    print(f"gemm_fp16 M={M} N={N} K={K}", flush=True)
+    px.launch_gemm(stream, px.GEMM_FP16, dA, dB, dC, M, N, K, 1.0, 0.0)
+    stream.synchronize()
+    a = oracle.f16_to_f32(np.uint16([0x3838]))[0]
+    want = oracle.f16_bits((a * B.sum(axis=0)).astype(np.float32))  # the sums are exact in f32
+    rows = 1 << 16
+    for r in [0, M // 3, 1 << 30, M - 5 * rows, M - rows]:
+        out = np.empty((rows, N), np.uint16)
+        px.check(px.lib().phx_memcpy_d2h(out.ctypes.data, dC.ptr + r * N * 2, out.nbytes))
+        assert (out == want.reshape(1, N)).all(), r
+    for b in (dA, dB, dC):
+        b.free()
