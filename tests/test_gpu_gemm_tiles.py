@@ -112,6 +112,51 @@ def test_each_tile_meets_the_oracle(px_gpu, stream, kern_name, M, N, K, pad):
     px.module_unload(mod)
 
 
+@pytest.mark.parametrize("chunk", [32, 96, 160])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 40), (65, 72, 200), (130, 136, 264), (200, 264, 328),
+                                   (257, 320, 1000)])
+@pytest.mark.parametrize("kern_name", [k for k in KERNELS if k != "MATMUL"])
+def test_each_split_form_meets_the_oracle(px_gpu, stream, kern_name, M, N, K, chunk):
+    # every split-K entry launched by itself over its own grid, then the reduce
+    # kernel: chunks of an odd number of 32 columns (a partial step of the 64
+    # deep tiles), the last one shorter, guard words behind the planes
+    px = px_gpu
+    case = _Case(px, getattr(px, kern_name), M, N, K, 8)
+    with open(os.path.join(px.LIB_DIR, KERNELS[kern_name][0]), "rb") as f:
+        mod = px.module_load_data(f.read())
+    reduce = px.module_get_function(mod, "gemm_splitk_reduce")
+    chunks = -(-K // chunk)
+    planes = chunks * M * N
+    guard = np.full(planes + 1024, 0x7FC00001, np.uint32)
+    ws = px.DeviceBuffer.from_array(guard)
+    i64, u64, u3 = ctypes.c_int64, ctypes.c_uint64, ctypes.c_uint32 * 3
+
+    def launch(fn, grid, vals):
+        arr = (ctypes.c_void_p * len(vals))(
+            *[ctypes.cast(ctypes.byref(v), ctypes.c_void_p) for v in vals])
+        px.check(px.lib().phx_launch(fn, u3(*grid), u3(256, 1, 1), 0, stream.handle, arr))
+
+    ld = [t.shape[1] for t in case.host]
+    for entry, (tm, tn) in KERNELS[kern_name][1].items():
+        ws.upload(guard)
+        case.dev[2].upload(case.host[2])
+        launch(px.module_get_function(mod, entry + "_splitk"),
+               (-(-M // tm) * -(-N // tn), chunks, 1),
+               [u64(case.dev[0].ptr), u64(case.dev[1].ptr), u64(ws.ptr)] +
+               [i64(x) for x in (ld[0], ld[1], M, N, K, chunk)])
+        launch(reduce, (-(-M * N // 1024), 1, 1),
+               [u64(ws.ptr), ctypes.c_int32(chunks), u64(case.dev[2].ptr), i64(ld[2]), i64(M),
+                i64(N), ctypes.c_float(0.75), ctypes.c_float(-0.5)])
+        stream.synchronize()
+        w = ws.download(np.uint32, planes + 1024)
+        assert (w[planes:] == guard[planes:]).all(), (entry, "store past the planes")
+        assert np.isfinite(w[:planes].view(np.float32)).all(), (entry, "plane not written")
+        out = case.dev[2].download(case.dt, case.host[2].shape)
+        assert np.array_equal(out[:, N:], case.host[2][:, N:]), (entry, "store outside C")
+        _check(case, out[:, :N].copy(), 0.75, -0.5)
+    px.module_unload(mod)
+
+
 @pytest.mark.parametrize("kern_name", list(KERNELS))
 @pytest.mark.parametrize("M,N,K", [(64, 64, 4096), (65, 72, 2056), (200, 520, 3000),
                                    (1000, 1000, 1000), (1208, 1208, 64), (300, 4096, 512),
