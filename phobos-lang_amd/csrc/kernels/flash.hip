@@ -861,12 +861,14 @@ extern "C" __global__ __launch_bounds__(256) void flash_combine(const float *W, 
             acc = acc * c;
             mx = m4;
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (s0 + u < nsplit) {  // uniform; no 0 * a: a may be infinite
-                    const float w = __builtin_amdgcn_exp2f(v[u].x - mx);
-                    l = l + w * v[u].y;
-                    acc = acc + w * a[u];
-                }
+            for (int u = 0; u < 4; ++u) {
+                const bool in = s0 + u < nsplit;
+                const float w = in ? __builtin_amdgcn_exp2f(v[u].x - mx) : 0.0f;
+                l = l + w * v[u].y;
+                // zeros, not 0 * a[u]: the sums may be infinite.  (A branch
+                // around them cost 0.3 us: the loads moved into it.)
+                acc = acc + w * (in ? a[u] : (phx_f4){0.0f, 0.0f, 0.0f, 0.0f});
+            }
         }
         const int64_t h = hqi / Nq, q = hqi % Nq;
         T *dst = O + h * ho + q * ldo + 4 * d4;
