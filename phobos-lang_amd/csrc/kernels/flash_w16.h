@@ -77,8 +77,10 @@ __device__ __forceinline__ void w16_step(Flash16 &fs, KFrag &kf, char *Vs, const
         fs.m2 = m2n;
     }
     fs.l += ps;
-    // V of block i landed: the loads of K and V a block later, 16 of them,
-    // were issued after it
+    // V of block i landed.  Issued after it: K and V of the group's next block,
+    // 16, and except in its last step (whose K loads nothing reads, so they
+    // are not there) K of the block after that; with those in flight, the wait
+    // for 16 is also one for the next block's K.
     __builtin_amdgcn_sched_barrier(0);
     PHX_WAIT_VMCNT(16);
     pv(fs.acc, Vs, pf, lane);
