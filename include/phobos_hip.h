@@ -173,8 +173,8 @@ int phx_check_shape(phx_kernel k, const int64_t *dims, int ndims);
  * split of the 256 x 256 tile and of the regular flash kernel, and the most a
  * launch uses: one that follows the built-in plan runs a smaller output tile
  * or a small-launch flash kernel instead, with fewer chunks or none, where
- * that is faster.  Other
- * kernels never split.  No counterpart in the reference, whose autotuner
+ * that is faster (which one, it decides by the workspace that is bound).
+ * Other kernels never split.  No counterpart in the reference, whose autotuner
  * picks tile sizes instead (phobos-bench/src/autotune.rs:98-192). */
 int phx_split_plan(phx_kernel k, const int64_t *dims, int ndims, int *splits,
                    size_t *workspace_bytes);
@@ -201,13 +201,18 @@ int phx_split_plan(phx_kernel k, const int64_t *dims, int ndims, int *splits,
  * (gemm_fp16tc_fp32acc and gemm_fp16: 64 x 64, 128 x 64 or 128 x 128, entries
  * "gemm_m64", "gemm_m128x64", "gemm_m128"; gemm_fp32: 64 x 64, 64 x 32 or 32 x
  * 32, entries "gemm_s64", "gemm_s64x32", "gemm_s32"; and their "_splitk"
- * forms); any other pin runs the tile it names.  The PHX_GEMM_SPLIT, PHX_FLASH_SPLIT and PHX_GEMM_W8 environment
- * variables, which force a plan for measurement, take precedence over both. */
+ * forms), never one whose f32 sums are less exact than the plan's own; flash
+ * launches likewise a small-launch kernel ("flash_w4", "flash_w2x4",
+ * "flash_w8").  Any other pin runs the tile it names.  The PHX_GEMM_SPLIT,
+ * PHX_FLASH_SPLIT and PHX_GEMM_W8 environment variables, which force a plan
+ * for measurement, take precedence over both. */
 typedef struct {
     int32_t splits;
     int32_t variant;
 } phx_plan;
-/* The plan a launch of k over dims (as phx_grid_for) would use now. */
+/* The plan of a launch of k over dims (as phx_grid_for) now: the pinned or
+ * built-in one.  Under the built-in one the launch may take a smaller tile or
+ * a small-launch flash kernel, as above, which no plan names. */
 int phx_plan_get(phx_kernel k, const int64_t *dims, int ndims, phx_plan *plan);
 /* Pins plan for k at dims (plan NULL removes the pin).  The one-head and
  * batched flash kernels of a precision share pins, the one-head dims meaning
@@ -291,7 +296,7 @@ int phx_arena_stats(phx_arena a, size_t *cap, size_t *bump, uint64_t *base);
  * PHX_SCRATCH_BYTES (16 MiB) device array that the library holds on each
  * initialised GPU until the process ends, instead of the stream's workspace
  * (it splits whether or not one is bound).  A split that needs more
- * scratch (phx_split_plan) returns PHX_E_INVALID; phx_flash_attention_bh
+ * scratch (phx_split_plan, whichever kernel would run) returns PHX_E_INVALID; phx_flash_attention_bh
  * takes any size.  Every call on a GPU
  * shares that GPU's array: calls that overlap on one GPU (several streams or
  * threads) race. */

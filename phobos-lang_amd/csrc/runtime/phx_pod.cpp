@@ -1257,10 +1257,11 @@ static int run_instrs(phx_pod p, std::vector<Instr> &ins, uint64_t stats[8]) {
             hipStream_t s = p->streams[p->next_stream];
             p->next_stream = (p->next_stream + 1) % p->streams.size();
             Inflight fl{Inflight::Kernel, i};
-            // A built-in GEMM or flash leaf too small to fill the GPU runs
+            // A built-in GEMM or flash leaf too small to fill the GPU may run
             // split; its partial results take an arena slab, as any tile
             // does (tile_store.rs:14-83), bound to the launch stream for this
-            // one launch.  When the arena cannot hold it the leaf runs unsplit.
+            // one launch: what its plan's chunks need, the most it uses.  When
+            // the arena cannot hold it the leaf runs unsplit.
             size_t ws_bytes = 0;
             if (kit != p->kernels.end()) {
                 const phx_kernel k = kit->second;
