@@ -674,9 +674,9 @@ static const HTile *gemm_tile_plan(phx_kernel k, int64_t M, int64_t N, int64_t K
             const int sp = want == 1 ? 1 : round_split(units, want);
             if (sp == last) continue;
             last = sp;
-            if (k != PHX_GEMM_FP16 && sum_noise(K, sp, tiles[i].sets, 1, 16) > noise) continue;
             const int64_t ns = htile_cost(tiles[i], M, N, K, sp);
-            if (!best || ns < least) {
+            if ((!best || ns < least) &&
+                (k == PHX_GEMM_FP16 || sum_noise(K, sp, tiles[i].sets, 1, 16) <= noise)) {
                 best = &tiles[i];
                 least = ns;
                 *splits = sp;
@@ -734,9 +734,8 @@ static const SHTile *s_tile_plan(int64_t M, int64_t N, int64_t K, int max_sp, in
             const int sp = want == 1 ? 1 : round_split(units, want);
             if (sp == last) continue;
             last = sp;
-            if (sum_noise(K, sp, ti.sets, ti.shares, 2) > noise) continue;
             const int64_t ns = stile_cost(ti, M, N, K, sp);
-            if (!best || ns < least) {
+            if ((!best || ns < least) && sum_noise(K, sp, ti.sets, ti.shares, 2) <= noise) {
                 best = &ti;
                 least = ns;
                 *splits = sp;
