@@ -200,8 +200,8 @@ int phx_split_plan(phx_kernel k, const int64_t *dims, int ndims, int *splits,
  * may run a smaller output tile with at most the rule's chunks
  * (gemm_fp16tc_fp32acc and gemm_fp16: 64 x 64, 128 x 64 or 128 x 128, entries
  * "gemm_m64", "gemm_m128x64", "gemm_m128"; gemm_fp32: 64 x 64, 64 x 32 or 32 x
- * 32, entries "gemm_s64", "gemm_s64x32", "gemm_s32"; and their "_splitk"
- * forms), never one whose f32 sums are less exact than the plan's own; flash
+ * 32, entries "gemm_s64", "gemm_s64x32", "gemm_s32" and "gemm_s32a4"; and the
+ * "_splitk" forms of all but the last), never one whose f32 sums are less exact than the plan's own; flash
  * launches likewise a small-launch kernel ("flash_w4", "flash_w2x4",
  * "flash_w8").  Any other pin runs the tile it names.  The PHX_GEMM_SPLIT,
  * PHX_FLASH_SPLIT and PHX_GEMM_W8 environment variables, which force a plan

@@ -392,6 +392,7 @@ typedef Tile<PHX_S_TILE, PHX_S_TILE, PHX_S_BK> Base;  // 256 x 256 x 16
 typedef STile<2, 2, 32> S64;
 typedef STile<2, 1, 32> S64x32;
 typedef STile<1, 1, 64> S32;
+typedef STile<1, 1, 64, 4> S32a4;
 
 #define GEMM_S_TILE_ENTRY(NAME, T, BETA)                                                      \
     extern "C" __global__ __launch_bounds__(NT, 3) void NAME(                                 \
@@ -407,6 +408,7 @@ typedef STile<1, 1, 64> S32;
 GEMM_S_TILE_ENTRY(gemm_s64, S64, beta)
 GEMM_S_TILE_ENTRY(gemm_s64x32, S64x32, beta)
 GEMM_S_TILE_ENTRY(gemm_s32, S32, beta)
+GEMM_S_TILE_ENTRY(gemm_s32a4, S32a4, beta)
 
 // Their split-K forms, as gemm_splitk below.
 #define GEMM_S_TILE_SPLIT(NAME, T)                                                            \

@@ -21,9 +21,15 @@
 
 // A TM x TN output tile per workgroup of 4 waves: WR x WC MFMA tiles of 32 x
 // 32, each of which KW = 4 / (WR WC) waves share, taking TK / KW of every K
-// step.  TK / KW = 16 or 32: 2 or 4 k-groups of 8 per wave and step.
-template <int WR_, int WC_, int TK_>
+// step.  TK / KW = 16 or 32: 2 or 4 k-groups of 8 per wave and step.  NA
+// accumulators in turn: two, since an MFMA that adds to the one before it waits
+// about 15 cycles more than its 64; four (gemm_s32a4) where the tile stands in
+// for a split of many chunks, whose chains of sums are that short (400 x 96 x
+// 376 against f64: 1.22e-7 in 12 chunks, 1.34e-7 with two, 1.06e-7 with four;
+// 512^3 runs in 5.41 us with four, 5.33 with two).
+template <int WR_, int WC_, int TK_, int NA_ = 2>
 struct STile {
+    static constexpr int NA = NA_;
     static constexpr int WR = WR_, WC = WC_, KW = 4 / (WR * WC), TK = TK_;
     static constexpr int TM = 32 * WR, TN = 32 * WC;
     static constexpr int AROW = TK * 4, BROW = TN * 4;      // LDS row bytes
@@ -132,11 +138,10 @@ __device__ __forceinline__ void s_body(const float *A, int64_t lda, const float 
                     vb[c - T::AC], 0, 0, 0);
         };
         constexpr int DMA = T::AC + T::BC, NM = 4 * T::NG;
-        // two accumulators in turn: an MFMA that adds to the one before it
-        // waits about 15 cycles more than its 64
-        phx_f16v acc[2];
-        acc[0] = (phx_f16v){0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-        acc[1] = acc[0];
+        phx_f16v acc[T::NA];
+#pragma unroll
+        for (int x = 0; x < T::NA; ++x)
+            acc[x] = (phx_f16v){0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
 #pragma unroll
@@ -163,8 +168,9 @@ __device__ __forceinline__ void s_body(const float *A, int64_t lda, const float 
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
                     const int m = 4 * g + s;
-                    acc[s & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(f[g & 1].a[s], f[g & 1].b[s],
-                                                                      acc[s & 1], 0, 0, 0);
+                    phx_f16v &c = acc[s % T::NA];
+                    c = __builtin_amdgcn_mfma_f32_32x32x2f32(f[g & 1].a[s], f[g & 1].b[s], c, 0, 0,
+                                                             0);
 #pragma unroll
                     for (int r = s * 5 / 4; r < (s + 1) * 5 / 4; ++r)
                         s_read<T>(f[(g + 1) & 1], last ? S[(u + 1) % 3] : S[u],
@@ -183,7 +189,10 @@ __device__ __forceinline__ void s_body(const float *A, int64_t lda, const float 
         }
         if (kt < nk) step(kt, 0);
         if (kt + 1 < nk) step(kt + 1, 1);
-        acc[0] = acc[0] + acc[1];
+#pragma unroll
+        for (int h = T::NA / 2; h > 0; h /= 2)  // pairwise
+#pragma unroll
+            for (int x = 0; x < h; ++x) acc[x] = acc[x] + acc[x + h];
 
         // Epilogue: the waves' sums to LDS as [wave][register][lane]; then the
         // KW waves of an MFMA tile take 32 / KW of its rows each, 8 lanes a

@@ -706,6 +706,9 @@ static const SHTile kSTiles[] = {
     {"gemm_s64", "gemm_s64_splitk", "matmul_s64", 64, 64, 2, 1, 800, {930, 1800, 2680}},
     {"gemm_s64x32", "gemm_s64x32_splitk", "matmul_s64x32", 64, 32, 2, 2, 600, {780, 1140, 1380}},
     {"gemm_s32", "gemm_s32_splitk", "matmul_s32", 32, 32, 2, 4, 550, {370, 560, 780}},
+    // where sum_noise rules out gemm_s32; unsplit, and never the leaf's (whose
+    // bound is one chain of K)
+    {"gemm_s32a4", nullptr, nullptr, 32, 32, 4, 4, 640, {370, 560, 780}},
 };
 // Workgroups a small f32 tile's launch starts at most, walking the tiles with
 // that stride: the three per CU that are resident at once (at 2048^3 the 64 x
@@ -730,7 +733,7 @@ static const SHTile *s_tile_plan(int64_t M, int64_t N, int64_t K, int max_sp, in
     const SHTile *best = nullptr;
     int64_t least = 0;
     for (const SHTile &ti : kSTiles)
-        for (int want = 1, last = 0; want <= max_sp; ++want) {
+        for (int want = 1, last = 0; want <= (ti.split_entry ? max_sp : 1); ++want) {
             const int sp = want == 1 ? 1 : round_split(units, want);
             if (sp == last) continue;
             last = sp;
